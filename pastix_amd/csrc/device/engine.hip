@@ -26,6 +26,7 @@
 #include "kernels_solve.hpp"
 #include "kernels_mfma.hpp"
 #include "kernels_svsolve.hpp"
+#include "kernels_panel.hpp"
 #include "pastix/kernels_enums.h"
 
 namespace {
@@ -44,7 +45,7 @@ struct level_t {
     int64_t m0, m1;     // one-wavefront solve tasks (levels whose cblks all fit one chunk, no Schur part)
     int64_t i0, i1;     // block-column inversion tasks
     int64_t g0, g1;     // blok updates (upd_group)
-    int64_t q0, q1;     // multi-workgroup panel tasks (32-row blocks of the diagonal tiles)
+    int64_t q0, q1, q2; // panel tasks: [q0, q1) rows of the diagonal tiles, [q1, q2) columns of their inverses
     int32_t maxn;
 };
 
@@ -226,8 +227,9 @@ struct pxd_ctx_s {
     // 1: panels, inverses, TRSM and the updates into the next level raise
     // their waves' issue priority (s_setprio) over the bulk updates
     int          prio = 1;
-    // 1: Cholesky diagonal tiles factored by one workgroup per 32-row block
-    // (k_potrf_mw); 0: one workgroup per cblk (k_potrf2)
+    // 1: Cholesky diagonal tiles factored and inverted by several workgroups
+    // (k_panel, as LDL^T and LU always are); 0: one workgroup per cblk
+    // (k_potrf2) and the inverses in a launch of their own (k_trtri)
     int          panel_mw = 1;
     // 1: the factorization runs one stream, launches every blok update on
     // its own and records per-workgroup times into model_entries
@@ -365,7 +367,7 @@ build_schedule( pxd_ctx_t *ctx )
     auto unfactored = [&]( int32_t k ) { return ctx->schur_fact_local && ctx->hcb[k].fcolnum >= ctx->schurfcol; };
 
     std::vector<int32_t>  list;
-    std::vector<pan_task> pan;
+    std::vector<pan_task> pan, pcol;
     std::vector<row_task> trsm, solv, diag;
     std::vector<inv_task> invt;
     std::vector<upd_task> upd, updb, upds;
@@ -419,6 +421,9 @@ build_schedule( pxd_ctx_t *ctx )
                 for ( int32_t pb = 0; pb < nblk; pb++ ) {
                     pan.push_back( pan_task{ k, pb, f0, nblk } );
                 }
+                for ( int32_t J = 0; J + 1 < nblk; J++ ) {
+                    pcol.push_back( pan_task{ k, J | PXD_PAN_COL, f0, nblk } );
+                }
             }
             for ( int32_t r0 = nk; r0 < c.stride; r0 += ctx->trsm_rt ) {
                 trsm.push_back( row_task{ k, r0 } );
@@ -427,6 +432,16 @@ build_schedule( pxd_ctx_t *ctx )
                 invt.push_back( inv_task{ k, J } );
             }
         }
+        // the columns wait for rows of this level only, which all precede them
+        lv.q1 = pan.size();
+        for ( int side = 0; side < ( lu ? 2 : 1 ); side++ ) {
+            for ( pan_task t : pcol ) {
+                t.p |= side ? PXD_PAN_USIDE : 0;
+                pan.push_back( t );
+            }
+        }
+        pcol.clear();
+        lv.q2 = pan.size();
         if ( lv.ds < 0 ) {
             lv.ds = diag.size();
             lv.fs = solv.size();
@@ -535,7 +550,6 @@ build_schedule( pxd_ctx_t *ctx )
             i = j;
         }
         lv.c1 = list.size();
-        lv.q1 = pan.size();
         lv.t1 = trsm.size();
         lv.u1 = upd.size();
         lv.b1 = updb.size();
@@ -636,8 +650,9 @@ ev_ms( hipEvent_t a, hipEvent_t b )
 }
 
 // Records of the kernel timing log from the workgroup stamps of one
-// factorization (layout of the stamp buffer: panels, inversions L and U
-// sides, TRSM tiles L and U sides, 64 x 64 update tiles, tall update tiles).
+// factorization (layout of the stamp buffer: panels with the columns of the
+// inverses, inversions of their own launch (panel_mw = 0), TRSM tiles L and U
+// sides, 64 x 64 update tiles, tall update tiles).
 // A panel is logged as (n, 0, 0) like cpucblk_zpotrfsp1d
 // (kernels/core_zpotrfsp.c:258); the TRSM of a cblk as (stride - n, n, 0) like
 // cpucblk_ztrsmsp (kernels/core_ztrsmsp.c:366-397), with its block-column
@@ -653,7 +668,7 @@ model_log_entries( pxd_ctx_t *ctx, const std::vector<uint64_t> &hs, int64_t n_li
     const int       nside = lu ? 2 : 1;
     const uint64_t *sp    = hs.data();
     const uint64_t *si    = sp + 2 * n_list;
-    const uint64_t *sm    = si + 4 * n_inv;
+    const uint64_t *sm    = si + 2 * n_inv;
     const uint64_t *su    = sm + 4 * n_trsm;
     const uint64_t *sb    = su + 2 * n_upd;
     const uint64_t *ss    = sb + 2 * n_updb;   // small updates: one task per launch in this mode
@@ -689,13 +704,19 @@ model_log_entries( pxd_ctx_t *ctx, const std::vector<uint64_t> &hs, int64_t n_li
     const int kpanel = lu ? PastixKernelGETRF : ( ctx->facto == FACT_SYTRF ) ? PastixKernelSYTRF : PastixKernelPOTRF;
     std::vector<pxd_model_entry_t> &out = ctx->model_entries;
     out.clear();
-    // multi-workgroup panels: the tasks of cblk k in the panel-task list
-    std::vector<int64_t> qb( nc + 1, 0 ), qe( nc + 1, 0 );
+    // multi-workgroup panels: the rows of cblk k and the columns of its
+    // inverses (both sides) in the panel-task list
+    std::vector<int64_t> qb[3], qe[3];
+    for ( int a = 0; a < 3; a++ ) {
+        qb[a].assign( nc + 1, 0 );
+        qe[a].assign( nc + 1, 0 );
+    }
     if ( mw ) {
         for ( int64_t i = (int64_t)ctx->hpan.size() - 1; i >= 0; i-- ) {
-            const int32_t k = ctx->hpan[i].cblk;
-            if ( qe[k] == 0 ) qe[k] = i + 1;
-            qb[k] = i;
+            const pan_task &t = ctx->hpan[i];
+            const int       a = !( t.p & PXD_PAN_COL ) ? 0 : ( t.p & PXD_PAN_USIDE ) ? 2 : 1;
+            if ( qe[a][t.cblk] == 0 ) qe[a][t.cblk] = i + 1;
+            qb[a][t.cblk] = i;
         }
     }
     for ( const level_t &lv : ctx->levels ) {
@@ -704,7 +725,7 @@ model_log_entries( pxd_ctx_t *ctx, const std::vector<uint64_t> &hs, int64_t n_li
             const dcblk  &c = ctx->hcb[k];
             const int32_t n = c.lcolnum - c.fcolnum + 1;
             double        t = 0.;
-            if ( mw ? span( sp, qb[k], qe[k], t ) : span( sp, i, i + 1, t ) ) {
+            if ( mw ? span( sp, qb[0][k], qe[0][k], t ) : span( sp, i, i + 1, t ) ) {
                 out.push_back( pxd_model_entry_t{ kpanel, n, 0, 0, t, -1, 0 } );
             }
             if ( c.stride == n ) {
@@ -712,7 +733,12 @@ model_log_entries( pxd_ctx_t *ctx, const std::vector<uint64_t> &hs, int64_t n_li
             }
             for ( int side = 0; side < nside; side++ ) {
                 double tt = 0.;
-                span( si + 2 * side * n_inv, ib[k], ie[k], tt );
+                if ( mw ) {
+                    span( sp, qb[1 + side][k], qe[1 + side][k], tt );
+                }
+                else {
+                    span( si, ib[k], ie[k], tt );
+                }
                 if ( span( sm + 2 * side * n_trsm, tb[k], te[k], tt ) ) {
                     out.push_back( pxd_model_entry_t{ PastixKernelTRSMCblk2d, c.stride - n, n, 0, tt, -1, 0 } );
                 }
@@ -783,11 +809,11 @@ factorize( pxd_ctx_t *ctx, double thresh, int64_t *nbpivots )
     }
 
     // kernel timing log: stamps of every panel, inversion, TRSM and update
-    // workgroup (LU: inversions and TRSM of both sides)
+    // workgroup (LU: TRSM of both sides)
     const bool mlog = ctx->model_log && ctx->kernels;
     uint64_t *stamps_all = nullptr, *st_panel = nullptr, *st_inv = nullptr, *st_trsm = nullptr;
     uint64_t *st_upd = nullptr, *st_updb = nullptr, *st_upds = nullptr;
-    const bool    use_mw = ctx->panel_mw && ctx->kernels && !lu && !ldlt;
+    const bool    use_mw = ctx->kernels && ( ctx->panel_mw || lu || ldlt );
     const int64_t n_list = use_mw ? (int64_t)ctx->hpan.size() : (int64_t)ctx->hlist.size();
     const int64_t n_inv = ctx->hinvt.size(), n_trsm = ctx->htrsm.size();
     int64_t n_upd = 0, n_updb = 0, n_upds = 0;
@@ -796,33 +822,30 @@ factorize( pxd_ctx_t *ctx, double thresh, int64_t *nbpivots )
         n_updb = std::max( n_updb, lv.b1 );
         n_upds = std::max( n_upds, lv.s1 );
     }
-    const int64_t n_st = n_list + 2 * n_inv + 2 * n_trsm + n_upd + n_updb + n_upds;
+    const int64_t n_st = n_list + n_inv + 2 * n_trsm + n_upd + n_updb + n_upds;
     if ( mlog ) {
         PXD_CHECK( hipMalloc( (void **)&stamps_all, 2 * sizeof( uint64_t ) * std::max<int64_t>( 1, n_st ) ) );
         PXD_CHECK( hipMemsetAsync( stamps_all, 0, 2 * sizeof( uint64_t ) * std::max<int64_t>( 1, n_st ), s ) );
         st_panel = stamps_all;
         st_inv   = st_panel + 2 * n_list;
-        st_trsm  = st_inv + 4 * n_inv;
+        st_trsm  = st_inv + 2 * n_inv;
         st_upd   = st_trsm + 4 * n_trsm;
         st_updb  = st_upd + 2 * n_upd;
         st_upds  = st_updb + 2 * n_updb;
     }
-    // rows of the panel's L21 strip and of the inverse's R block kept in
-    // LDS (PXD_NB + 1 values each); the kernels keep the rest in HBM
-    const size_t  lds_row = ( PXD_NB + 1 ) * sizeof( T );
-    const void   *potrf2  = (const void *)k_potrf2<T, true>;
-    if constexpr ( std::is_same<T, typename px_real<T>::type>::value ) {
-        if ( !ldlt ) {
-            potrf2 = (const void *)k_potrf2<T, false>;
+    // rows of the one-workgroup panel's L21 strip and of the inverse's R
+    // block kept in LDS (PXD_NB + 1 values each); the kernels keep the rest in HBM
+    const size_t lds_row = ( PXD_NB + 1 ) * sizeof( T );
+    int32_t      pcap = 0, rcap = 0;
+    if constexpr ( std::is_same<T, R>::value ) {
+        pcap = (int32_t)( lds_room( (const void *)k_potrf2<T>, ctx->lds_max ) / lds_row );
+        rcap = (int32_t)( lds_room( (const void *)k_trtri<T>, ctx->lds_max ) / lds_row );
+        if ( ctx->kernels && !use_mw && ( rcap < 1 || pcap < 1 ) ) {
+            if ( stamps_all ) {
+                (void)hipFree( stamps_all );
+            }
+            return 3;
         }
-    }
-    const int32_t pcap = (int32_t)( lds_room( potrf2, ctx->lds_max ) / lds_row );
-    const int32_t rcap = (int32_t)( lds_room( (const void *)k_trtri<T>, ctx->lds_max ) / lds_row );
-    if ( ctx->kernels && ( rcap < 1 || ( !lu && pcap < 1 ) ) ) {
-        if ( stamps_all ) {
-            (void)hipFree( stamps_all );
-        }
-        return 3;
     }
     // stamps of the tasks [i0, ...) of a launch (side 1: the U side's copy)
     auto stp = [&]( uint64_t *base, int64_t i0, int side, int64_t nside ) -> uint64_t * {
@@ -844,53 +867,62 @@ factorize( pxd_ctx_t *ctx, double thresh, int64_t *nbpivots )
         if ( np == 0 ) {
             return;   // a level of unfactored Schur cblks only
         }
-        // rows below a block column of the widest cblk of the level
-        const size_t trtri_lds = (size_t)std::max( 1, std::min( lv.maxn - PXD_NB, rcap ) ) * lds_row;
-        if ( lu ) {
-            hipLaunchKernelGGL( ( k_getrf2<T> ), dim3( np ), dim3( PXD_THREADS ), 0, st, ctx->dlist + lv.c0,
-                                ctx->dcb, L, U, DI, DU, thresh, ctx->dscratch, stp( st_panel, lv.c0, 0, 0 ), ctx->prio );
-            launches++;
-            if ( ni ) {
-                hipLaunchKernelGGL( ( k_trtri<T> ), dim3( ni ), dim3( PXD_THREADS ), trtri_lds, st,
-                                    ctx->dinvt + lv.i0, ctx->dcb, (const T *)L, DI, stp( st_inv, lv.i0, 0, n_inv ), ctx->prio, rcap );
-                hipLaunchKernelGGL( ( k_trtri<T> ), dim3( ni ), dim3( PXD_THREADS ), trtri_lds, st,
-                                    ctx->dinvt + lv.i0, ctx->dcb, (const T *)U, DU, stp( st_inv, lv.i0, 1, n_inv ), ctx->prio, rcap );
-                launches += 2;
+        if ( use_mw ) {
+            // the rows of the tiles and the columns of their inverses in one
+            // launch; the timing log takes them one after the other, so that
+            // a column's time holds no waiting for its rows
+            auto rows = [&]( int64_t q0, int64_t q1 ) {
+                const dim3 grid( (unsigned)( q1 - q0 ) );
+                uint64_t  *sp = stp( st_panel, q0, 0, 0 );
+                if ( q0 == q1 ) {
+                    return;
+                }
+                if ( lu ) {
+                    hipLaunchKernelGGL( ( k_panel<T, PAN_LU> ), grid, dim3( PXD_THREADS ), 0, st, ctx->dpan + q0,
+                                        ctx->dcb, L, U, DI, DU, thresh, ctx->dscratch, ctx->dflags, ctx->dscratch + 2,
+                                        sp, ctx->prio );
+                }
+                else if ( ldlt ) {
+                    hipLaunchKernelGGL( ( k_panel<T, PAN_LDLT> ), grid, dim3( PXD_THREADS ), 0, st, ctx->dpan + q0,
+                                        ctx->dcb, L, L, DI, DI, thresh, ctx->dscratch, ctx->dflags, ctx->dscratch + 2,
+                                        sp, ctx->prio );
+                }
+                else if constexpr ( std::is_same<T, R>::value ) {
+                    hipLaunchKernelGGL( ( k_panel<T, PAN_LLT> ), grid, dim3( PXD_THREADS ), 0, st, ctx->dpan + q0,
+                                        ctx->dcb, L, L, DI, DI, thresh, ctx->dscratch, ctx->dflags, ctx->dscratch + 2,
+                                        sp, ctx->prio );
+                }
+                launches++;
+            };
+            if ( mlog ) {
+                rows( lv.q0, lv.q1 );
+                rows( lv.q1, lv.q2 );
+            }
+            else {
+                rows( lv.q0, lv.q2 );
             }
         }
-        else if ( ctx->kernels ) {
-            const size_t sh = (size_t)std::max( 1, std::min( lv.maxn, pcap ) ) * lds_row;
-            if ( ldlt ) {
-                hipLaunchKernelGGL( ( k_potrf2<T, true> ), dim3( np ), dim3( PXD_THREADS ), sh, st, ctx->dlist + lv.c0,
-                                    ctx->dcb, L, DI, thresh, ctx->dscratch, stp( st_panel, lv.c0, 0, 0 ), ctx->prio, pcap );
-            }
-            else if constexpr ( std::is_same<T, R>::value ) {
-                if ( ctx->panel_mw ) {
-                    // one workgroup per 32-row block of each diagonal tile
-                    const unsigned nq  = (unsigned)( lv.q1 - lv.q0 );
-                    const size_t   shq = (size_t)( ( std::max( 1, lv.maxn ) + PXD_NB - 1 ) / PXD_NB ) * PXD_NB *
-                                       ( PXD_NB + 1 ) * sizeof( T );
-                    hipLaunchKernelGGL( ( k_potrf_mw<T> ), dim3( nq ), dim3( PXD_THREADS ), shq, st,
-                                        ctx->dpan + lv.q0, ctx->dcb, L, DI, thresh, ctx->dscratch, ctx->dflags,
-                                        ctx->dscratch + 2, stp( st_panel, lv.q0, 0, 0 ), ctx->prio );
-                }
-                else {
-                    hipLaunchKernelGGL( ( k_potrf2<T, false> ), dim3( np ), dim3( PXD_THREADS ), sh, st,
-                                        ctx->dlist + lv.c0, ctx->dcb, L, DI, thresh, ctx->dscratch,
-                                        stp( st_panel, lv.c0, 0, 0 ), ctx->prio, pcap );
+        else if constexpr ( std::is_same<T, R>::value ) {
+            if ( ctx->kernels ) {
+                // rows below a block column of the widest cblk of the level
+                const size_t trtri_lds = (size_t)std::max( 1, std::min( lv.maxn - PXD_NB, rcap ) ) * lds_row;
+                const size_t sh        = (size_t)std::max( 1, std::min( lv.maxn, pcap ) ) * lds_row;
+                hipLaunchKernelGGL( ( k_potrf2<T> ), dim3( np ), dim3( PXD_THREADS ), sh, st, ctx->dlist + lv.c0,
+                                    ctx->dcb, L, DI, thresh, ctx->dscratch, stp( st_panel, lv.c0, 0, 0 ), ctx->prio,
+                                    pcap );
+                launches++;
+                if ( ni ) {
+                    hipLaunchKernelGGL( ( k_trtri<T> ), dim3( ni ), dim3( PXD_THREADS ), trtri_lds, st,
+                                        ctx->dinvt + lv.i0, ctx->dcb, (const T *)L, DI, stp( st_inv, lv.i0, 0, 0 ),
+                                        ctx->prio, rcap );
+                    launches++;
                 }
             }
-            launches++;
-            if ( ni ) {
-                hipLaunchKernelGGL( ( k_trtri<T> ), dim3( ni ), dim3( PXD_THREADS ), trtri_lds, st,
-                                    ctx->dinvt + lv.i0, ctx->dcb, (const T *)L, DI, stp( st_inv, lv.i0, 0, n_inv ), ctx->prio, rcap );
+            else {
+                hipLaunchKernelGGL( ( k_potrf<T> ), dim3( np ), dim3( PXD_THREADS ), 0, st, ctx->dlist + lv.c0,
+                                    ctx->dcb, L, DI, thresh, ctx->dscratch );
                 launches++;
             }
-        }
-        else if constexpr ( std::is_same<T, typename px_real<T>::type>::value ) {
-            hipLaunchKernelGGL( ( k_potrf<T> ), dim3( np ), dim3( PXD_THREADS ), 0, st, ctx->dlist + lv.c0,
-                                ctx->dcb, L, DI, thresh, ctx->dscratch );
-            launches++;
         }
     };
     auto trsm = [&]( const level_t &lv, hipStream_t st ) {
@@ -1405,11 +1437,9 @@ void
 set_lds_attributes_mfma( size_t lds )
 {
     if constexpr ( std::is_same<T, typename px_real<T>::type>::value ) {
-        set_lds_room( (const void *)k_potrf2<T, false>, lds );
-        set_lds_room( (const void *)k_potrf_mw<T>, lds );
+        set_lds_room( (const void *)k_potrf2<T>, lds );
+        set_lds_room( (const void *)k_trtri<T>, lds );
     }
-    set_lds_room( (const void *)k_potrf2<T, true>, lds );
-    set_lds_room( (const void *)k_trtri<T>, lds );
     set_lds_attributes_solve<T, T>( lds );
 }
 

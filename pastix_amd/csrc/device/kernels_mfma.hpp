@@ -407,10 +407,11 @@ search_grow( const search_keys &sk, const dblok *__restrict__ bk, int32_t ffb, i
 // PXD_NB columns; the unblocked step updates with unscaled columns so that it
 // needs one barrier per column.  The inverses of the PXD_NB x PXD_NB diagonal
 // sub-blocks go to the diagonal blocks of Linv.  The first pcap rows of the
-// current block's L21 are kept in dynamic LDS; rows beyond pcap (wide cblks in
-// complex double, whose strip would not fit the CU's LDS) are read back from
-// the copy just written to A.
-template <typename T, bool LDLT>
+// current block's L21 are kept in dynamic LDS; rows beyond pcap (a strip that
+// would not fit the CU's LDS) are read back from the copy just written to A.
+// Option panel_mw = 0: one workgroup per cblk, where k_panel takes one per
+// 32-row block.
+template <typename T>
 __global__ void __launch_bounds__( PXD_THREADS )
 k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__restrict__ L,
           T *__restrict__ Linv, double thresh, int *__restrict__ npiv,
@@ -419,7 +420,6 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
     __shared__ T sA[PXD_NB][PXD_NB + 1];   // sA[col][row]
     __shared__ T sI[PXD_NB][PXD_NB + 1];   // inverse, sI[col][row]
     __shared__ T sD[PXD_NB];
-    __shared__ T sDi[PXD_NB];               // LDL^T: 1 / D of the block, 0 beyond it
     __shared__ T sX[4][PXD_NB];             // exchange area of the elimination
     // L21 of the current block, sP[row][k]: dynamic LDS for the widest cblk of the launch
     extern __shared__ unsigned char smem_raw[];
@@ -458,48 +458,29 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
         __syncthreads();
 
         // unblocked elimination A = U D U^T, W = U^{-1} alongside
-        piv += elim_sym32<T, LDLT>( sA, sI, sD, sX, bs, tau, tid );
+        piv += elim_sym32<T, false>( sA, sI, sD, sX, bs, tau, tid );
         // Cholesky: L = U D^{1/2}, the columns scaled by 1/sqrt(pivot), and
-        // L^{-1} = D^{-1/2} U^{-1}, the rows of W scaled likewise.  LDL^T:
-        // L = U (column / d), L^{-1} = W, the diagonal holds D and the upper
-        // part D L^T (the unscaled columns).
+        // L^{-1} = D^{-1/2} U^{-1}, the rows of W scaled likewise.
         for ( int idx = tid; idx < PXD_NB * PXD_NB; idx += PXD_THREADS ) {
             const int rr = idx % PXD_NB, cc = idx / PXD_NB;
             if ( rr >= bs || cc >= bs ) continue;
             if ( rr > cc ) {
-                const T a = sA[cc][rr];
-                if constexpr ( LDLT ) {
-                    sA[rr][cc] = a;
-                    sA[cc][rr] = a / sD[cc];
-                }
-                else {
-                    sA[cc][rr] = a / px_sqrt( sD[cc] );
-                }
+                sA[cc][rr] = sA[cc][rr] / px_sqrt( sD[cc] );
             }
-            if constexpr ( !LDLT ) {
-                if ( rr >= cc ) {
-                    sI[cc][rr] = sI[cc][rr] / px_sqrt( sD[rr] );
-                }
+            if ( rr >= cc ) {
+                sI[cc][rr] = sI[cc][rr] / px_sqrt( sD[rr] );
             }
         }
         __syncthreads();
         if ( tid < bs ) {
-            if constexpr ( LDLT ) {
-                sA[tid][tid] = sD[tid];
-            }
-            else {
-                sA[tid][tid] = px_sqrt( sD[tid] );
-            }
-        }
-        if ( tid < PXD_NB ) {
-            sDi[tid] = ( tid < bs ) ? (T)1 / sD[tid] : (T)0;
+            sA[tid][tid] = px_sqrt( sD[tid] );
         }
         __syncthreads();
 
         for ( int idx = tid; idx < PXD_NB * PXD_NB; idx += PXD_THREADS ) {
             const int rr = idx % PXD_NB, cc = idx / PXD_NB;
             if ( rr >= bs || cc >= bs ) continue;
-            if ( LDLT || rr >= cc ) {
+            if ( rr >= cc ) {
                 A[( kb + rr ) + (int64_t)( kb + cc ) * n] = sA[cc][rr];
             }
             LI[( kb + rr ) + (int64_t)( kb + cc ) * n] = sI[cc][rr];
@@ -534,19 +515,12 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
                 const int32_t rr = rb + M::row( lane, v );
                 const int     c0 = lane & 15, c1 = 16 + ( lane & 15 );
                 if ( rr < m ) {
-                    // LDL^T: the product is L21 D; L21 = product / D goes below
-                    // the block and the product itself, transposed, to the
-                    // block's rows right of it (D L^T, core_zsytrfsp.c:176-186)
                     if ( rr < pcap ) {
                         sP[rr][c0] = M::get( acc0, v );   // zero beyond bs: sI is zero there
                         sP[rr][c1] = M::get( acc1, v );
                     }
-                    if ( c0 < bs ) A[( m0 + rr ) + (int64_t)( kb + c0 ) * n] = LDLT ? M::get( acc0, v ) * sDi[c0] : M::get( acc0, v );
-                    if ( c1 < bs ) A[( m0 + rr ) + (int64_t)( kb + c1 ) * n] = LDLT ? M::get( acc1, v ) * sDi[c1] : M::get( acc1, v );
-                    if constexpr ( LDLT ) {
-                        if ( c0 < bs ) A[( kb + c0 ) + (int64_t)( m0 + rr ) * n] = M::get( acc0, v );
-                        if ( c1 < bs ) A[( kb + c1 ) + (int64_t)( m0 + rr ) * n] = M::get( acc1, v );
-                    }
+                    if ( c0 < bs ) A[( m0 + rr ) + (int64_t)( kb + c0 ) * n] = M::get( acc0, v );
+                    if ( c1 < bs ) A[( m0 + rr ) + (int64_t)( kb + c1 ) * n] = M::get( acc1, v );
                 }
             }
         }
@@ -555,8 +529,7 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
         // trailing update A22 -= L21 L21^T (lower part) on the matrix cores
         // from sP: 32 x 32 tiles, wave w takes every fourth tile, two at a
         // time, with the tiles' loads of A22 issued before their products.
-        // Row ri of the product (L21, times D for LDL^T) beyond pcap comes
-        // from A: the D L^T strip for LDL^T, the L21 column block otherwise.
+        // Row ri of the product beyond pcap comes from A.
         auto prow = [&]( int32_t ri, int l ) -> T {
             if ( ri < pcap ) {
                 return sP[ri][l];
@@ -564,7 +537,7 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
             if ( l >= bs ) {
                 return (T)0;
             }
-            return LDLT ? A[( kb + l ) + (int64_t)( m0 + ri ) * n] : A[( m0 + ri ) + (int64_t)( kb + l ) * n];
+            return A[( m0 + ri ) + (int64_t)( kb + l ) * n];
         };
         {
             const int32_t nt = ( m + 31 ) / 32;
@@ -612,8 +585,7 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
                         for ( int a = 0; a < 2; a++ ) {
                             const int32_t ri = 32 * ti[g] + 16 * a + ( lane & 15 );
                             const int32_t rj = 32 * tj[g] + 16 * a + ( lane & 15 );
-                            // LDL^T: A22 -= (L21 D) D^{-1} (L21 D)^T
-                            af[a] = ( ri < m ) ? ( LDLT ? prow( ri, l ) * sDi[l] : prow( ri, l ) ) : (T)0;
+                            af[a] = ( ri < m ) ? prow( ri, l ) : (T)0;
                             bf[a] = ( rj < m ) ? prow( rj, l ) : (T)0;
                         }
 #pragma unroll
@@ -639,508 +611,6 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
             }
         }
         __syncthreads();
-    }
-    if ( tid == 0 && piv > 0 ) {
-        atomicAdd( npiv, piv );
-    }
-    stamp_end( stamps, blockIdx.x, t_stamp );
-}
-
-// ---------------------------------------------------------------------------
-// Multi-workgroup Cholesky of the diagonal tiles.  Task {cblk, p, flag0}:
-// the workgroup owns the 32-row block p of the cblk's n x n diagonal tile,
-// i.e. the 32 x 32 tiles T(p, 0..p), kept in LDS from the start.  For
-// k = 0..p-1 it waits until block k has factored its diagonal tile
-// (flag[k] > k), forms L(p,k) = T(p,k) L(k,k)^{-T} with the inverse that
-// block k wrote to Linv, publishes it (flag[p] = k+1), and subtracts
-// L(p,k) L(j,k)^T from its tiles T(p,j), j = k+1..p, each L(j,k) once
-// block j has published it.  For k = p it factors T(p,p) like one block of
-// k_potrf2 (static pivot, inverse built by the elimination) and publishes
-// flag[p] = p+1.  The critical path is the chain of diagonal tiles instead
-// of the n/32 sequential block steps of a single workgroup.
-//
-// Exchange between the workgroups: the L(p,k) tiles and the diagonal
-// inverses that other blocks read are written and read with agent-scope
-// relaxed atomic stores and loads (panel_st, panel_ld), which are coherent
-// across the XCDs by themselves.  Publication: every thread waits until its
-// own stores are complete, a barrier, then thread 0 stores the flag.  Waits:
-// thread 0 polls the flag, then a barrier.  No agent-scope fence is needed,
-// and none is issued: such a fence writes back (release) or invalidates
-// (acquire) the XCD's whole L2, which the update kernels of the other
-// stream keep filling (100^3: FP32 numfact 86.3 -> 85.4 ms).  Every wait is
-// bounded by a wall-clock deadline; on expiry the kernel records it in *err
-// and goes on, so every wave reaches the end.
-struct pan_task {
-    int32_t cblk;
-    int32_t p;
-    int32_t flag0;
-    int32_t nblk;    // blocks of the tile: the last one has no consumer
-};
-// Bound of one wait in ticks of the constant clock (wall_clock64), set on
-// every device from its clock rate when an engine context is created (2 s
-// by default, engine option "wait_ms").
-__constant__ uint64_t pxd_wait_ticks = 200000000ull;
-
-__device__ inline void
-panel_wait( const int *f, int target, int *err, int tid )
-{
-    if ( tid == 0 ) {
-        // after one timeout anywhere every later wait falls through at once
-        const uint64_t t0 = (uint64_t)wall_clock64();
-        while ( __hip_atomic_load( f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) < target &&
-                __hip_atomic_load( err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) == 0 ) {
-            if ( (uint64_t)wall_clock64() - t0 > pxd_wait_ticks ) {
-                __hip_atomic_store( err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
-                break;
-            }
-            __builtin_amdgcn_s_sleep( 1 );
-        }
-    }
-    __syncthreads();
-    __atomic_signal_fence( __ATOMIC_SEQ_CST );   // the block's loads stay after the wait
-}
-
-__device__ inline void
-panel_publish( int *f, int value, int tid )
-{
-    // each thread's panel_st stores complete (vmcnt 0) before the barrier,
-    // so the flag is stored after all of them
-    __atomic_signal_fence( __ATOMIC_SEQ_CST );
-    __builtin_amdgcn_s_waitcnt( 0 );
-    __syncthreads();
-    if ( tid == 0 ) {
-        __hip_atomic_store( f, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
-    }
-}
-
-// Loads and stores of the data that the panel's workgroups exchange.
-template <typename T>
-__device__ inline T
-panel_ld( const T *p )
-{
-    return __hip_atomic_load( p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
-}
-template <typename T>
-__device__ inline void
-panel_st( T *p, T v )
-{
-    __hip_atomic_store( p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
-}
-
-// P[r][c] = sum_l X[r][l] Y[c][l] for 32 x 32 tiles held as s[col][row]:
-// wave w computes the 16 x 16 quadrant (w >> 1, w & 1) on the matrix cores.
-template <typename T>
-__device__ inline typename mfma16<T>::acc_t
-tile_xyt( const T ( *sX )[PXD_NB + 1], const T ( *sY )[PXD_NB + 1], int lane, int w )
-{
-    typedef mfma16<T> M;
-    typename M::acc_t acc = M::zero();
-    const int qr = w >> 1, qc = w & 1;
-#pragma unroll
-    for ( int s4 = 0; s4 < PXD_NB / 4; s4++ ) {
-        const int l = 4 * s4 + ( lane >> 4 );
-        acc = M::mma( sX[l][16 * qr + ( lane & 15 )], sY[l][16 * qc + ( lane & 15 )], acc );
-    }
-    return acc;
-}
-
-template <typename T>
-__global__ void __launch_bounds__( PXD_THREADS )
-k_potrf_mw( const pan_task *__restrict__ tasks, const dcblk *__restrict__ cb, T *__restrict__ L,
-            T *__restrict__ Linv, double thresh, int *__restrict__ npiv, int *flags, int *err,
-            uint64_t *__restrict__ stamps, int prio )
-{
-    typedef mfma16<T>         M;
-    typedef typename M::acc_t acc_t;
-    typedef T                 tile_t[PXD_NB][PXD_NB + 1];   // [col][row]
-    __shared__ tile_t sI;                // inverse of a diagonal block
-    __shared__ tile_t sO;                // L(j,k) of another block
-    __shared__ T      sD[PXD_NB];
-    extern __shared__ unsigned char smem_raw[];
-    tile_t *sT = reinterpret_cast<tile_t *>( smem_raw );   // T(p, 0..p)
-
-    const pan_task tk      = tasks[blockIdx.x];
-    const uint64_t t_stamp = stamp_begin( stamps );
-    wave_priority( prio );
-    const dcblk   c    = cb[tk.cblk];
-    const int32_t n    = c.lcolnum - c.fcolnum + 1;
-    const int     p    = tk.p;
-    const int32_t R0   = PXD_NB * p;
-    const int32_t bs   = min( PXD_NB, n - R0 );
-    const int     tid  = threadIdx.x;
-    const int     lane = tid & 63, w = tid >> 6;
-    T            *A    = L + c.coefoff;
-    T            *LI   = Linv + c.dinvoff;
-    int          *flag = flags + tk.flag0;
-    const bool    last = ( p == tk.nblk - 1 );   // nobody waits for the last block
-    constexpr int NU   = PXD_NB * PXD_NB / PXD_THREADS;
-    int           piv  = 0;
-    typedef typename px_real<T>::type R;
-    const R tau = (R)thresh;
-
-    // the block row: T(p, j) for j = 0..p (lower part only for j = p).
-    // Every load is issued, the entries outside read a clamped in-range
-    // address and are masked: a load under its own branch made the compiler
-    // wait for the previous one.
-    for ( int j0 = 0; j0 <= p; j0 += 4 ) {
-        T v[4][NU];
-#pragma unroll
-        for ( int jj = 0; jj < 4; jj++ )
-#pragma unroll
-            for ( int u = 0; u < NU; u++ ) {
-                const int idx = tid + u * PXD_THREADS, r = idx % PXD_NB, cc = idx / PXD_NB, j = j0 + jj;
-                const bool    ok  = j <= p && r < bs && ( j < p || cc <= r );
-                const int32_t col = min( PXD_NB * min( j, p ) + cc, n - 1 );
-                const T       x   = A[( R0 + min( r, bs - 1 ) ) + (int64_t)col * n];
-                v[jj][u] = ok ? x : (T)0;
-            }
-#pragma unroll
-        for ( int jj = 0; jj < 4; jj++ )
-#pragma unroll
-            for ( int u = 0; u < NU; u++ ) {
-                const int idx = tid + u * PXD_THREADS, r = idx % PXD_NB, cc = idx / PXD_NB;
-                if ( j0 + jj <= p ) sT[j0 + jj][cc][r] = v[jj][u];
-            }
-    }
-
-    for ( int k = 0; k < p; k++ ) {
-        // L(p,k) = T(p,k) L(k,k)^{-T}
-        panel_wait( flag + k, k + 1, err, tid );
-        {
-            T v[NU];
-#pragma unroll
-            for ( int u = 0; u < NU; u++ ) {
-                const int idx = tid + u * PXD_THREADS, r = idx % PXD_NB, cc = idx / PXD_NB;
-                v[u] = panel_ld( LI + ( PXD_NB * k + r ) + (int64_t)( PXD_NB * k + cc ) * n );
-            }
-#pragma unroll
-            for ( int u = 0; u < NU; u++ ) {
-                const int idx = tid + u * PXD_THREADS, r = idx % PXD_NB, cc = idx / PXD_NB;
-                sI[cc][r] = v[u];
-            }
-        }
-        __syncthreads();
-        {
-            acc_t acc = tile_xyt<T>( sT[k], sI, lane, w );
-            __syncthreads();   // every wave has read T(p,k)
-            const int qr = w >> 1, qc = w & 1;
-#pragma unroll
-            for ( int v = 0; v < 4; v++ ) {
-                const int r = 16 * qr + M::row( lane, v ), cc = 16 * qc + ( lane & 15 );
-                const T   x = ( r < bs ) ? M::get( acc, v ) : (T)0;
-                sT[k][cc][r] = x;
-                if ( r < bs ) panel_st( A + ( R0 + r ) + (int64_t)( PXD_NB * k + cc ) * n, x );
-            }
-        }
-        if ( !last ) {
-            panel_publish( flag + p, k + 1, tid );
-        }
-        __syncthreads();   // sT[k] complete for every wave
-        // T(p,j) -= L(p,k) L(j,k)^T, j = k+1..p
-        for ( int j = k + 1; j <= p; j++ ) {
-            const tile_t *Y = &sT[k];
-            if ( j < p ) {
-                panel_wait( flag + j, k + 1, err, tid );
-                T v[NU];
-#pragma unroll
-                for ( int u = 0; u < NU; u++ ) {
-                    const int idx = tid + u * PXD_THREADS, r = idx % PXD_NB, cc = idx / PXD_NB;
-                    v[u] = panel_ld( A + ( PXD_NB * j + r ) + (int64_t)( PXD_NB * k + cc ) * n );
-                }
-#pragma unroll
-                for ( int u = 0; u < NU; u++ ) {
-                    const int idx = tid + u * PXD_THREADS, r = idx % PXD_NB, cc = idx / PXD_NB;
-                    sO[cc][r] = v[u];
-                }
-                __syncthreads();
-                Y = &sO;
-            }
-            acc_t     acc = tile_xyt<T>( sT[k], *Y, lane, w );
-            const int qr = w >> 1, qc = w & 1;
-#pragma unroll
-            for ( int v = 0; v < 4; v++ ) {
-                const int r = 16 * qr + M::row( lane, v ), cc = 16 * qc + ( lane & 15 );
-                sT[j][cc][r] -= M::get( acc, v );
-            }
-            __syncthreads();   // sO is reused by the next j
-        }
-    }
-
-    // T(p,p): elimination with the inverse built alongside (as in k_potrf2);
-    // sO is free now and serves as the exchange area
-    T( *sA )[PXD_NB + 1] = sT[p];
-    for ( int idx = tid; idx < PXD_NB * PXD_NB; idx += PXD_THREADS ) {
-        const int r = idx % PXD_NB, cc = idx / PXD_NB;
-        sI[cc][r] = ( r == cc && r < bs ) ? (T)1 : (T)0;
-    }
-    __syncthreads();
-    piv += elim_sym32<T, false>( sA, sI, sD, reinterpret_cast<T ( * )[PXD_NB]>( &sO[0][0] ), bs, tau, tid );
-    for ( int idx = tid; idx < PXD_NB * PXD_NB; idx += PXD_THREADS ) {
-        const int rr = idx % PXD_NB, cc = idx / PXD_NB;
-        if ( rr >= bs || cc >= bs ) continue;
-        if ( rr > cc ) {
-            sA[cc][rr] = sA[cc][rr] / px_sqrt( sD[cc] );
-        }
-        if ( rr >= cc ) {
-            sI[cc][rr] = sI[cc][rr] / px_sqrt( sD[rr] );
-        }
-    }
-    __syncthreads();
-    if ( tid < bs ) {
-        sA[tid][tid] = px_sqrt( sD[tid] );
-    }
-    __syncthreads();
-    for ( int idx = tid; idx < PXD_NB * PXD_NB; idx += PXD_THREADS ) {
-        const int rr = idx % PXD_NB, cc = idx / PXD_NB;
-        if ( rr >= bs || cc >= bs ) continue;
-        if ( rr >= cc ) {
-            A[( R0 + rr ) + (int64_t)( R0 + cc ) * n] = sA[cc][rr];
-        }
-        panel_st( LI + ( R0 + rr ) + (int64_t)( R0 + cc ) * n, sI[cc][rr] );
-    }
-    if ( !last ) {
-        panel_publish( flag + p, p + 1, tid );
-    }
-    if ( tid == 0 && piv > 0 ) {
-        atomicAdd( npiv, piv );
-    }
-    stamp_end( stamps, blockIdx.x, t_stamp );
-}
-
-// ---------------------------------------------------------------------------
-// X = B * S^T for a rows x 32 block B of the diagonal tile, in place, on the
-// matrix cores: wave w takes 16-row blocks w, w+4, ...; row i of B is
-// element (i, k) at base + i * rs + k * ks; S is a 32 x 32 matrix in LDS,
-// S[row][col] = sS[col][row].  Only the first bs columns of B are read or
-// written (S is zero outside its bs x bs corner).
-template <typename T>
-__device__ inline void
-small_trsm_mfma( T *base, int64_t rs, int64_t ks, int32_t rows, int32_t bs, const T ( *sS )[PXD_NB + 1],
-                 int tid )
-{
-    typedef mfma16<T>         M;
-    typedef typename M::acc_t acc_t;
-    const int lane = tid & 63, w = tid >> 6;
-    for ( int32_t rb = 16 * w; rb < rows; rb += 64 ) {
-        T             a[PXD_NB / 4];
-        const int32_t ra = rb + ( lane & 15 );
-#pragma unroll
-        for ( int s4 = 0; s4 < PXD_NB / 4; s4++ ) {
-            const int l = 4 * s4 + ( lane >> 4 );
-            a[s4] = ( ra < rows && l < bs ) ? base[ra * rs + l * ks] : (T)0;
-        }
-        acc_t acc0 = M::zero(), acc1 = M::zero();
-#pragma unroll
-        for ( int s4 = 0; s4 < PXD_NB / 4; s4++ ) {
-            const int l = 4 * s4 + ( lane >> 4 );
-            acc0 = M::mma( a[s4], sS[l][( lane & 15 )], acc0 );
-            acc1 = M::mma( a[s4], sS[l][16 + ( lane & 15 )], acc1 );
-        }
-#pragma unroll
-        for ( int v = 0; v < 4; v++ ) {
-            const int32_t rr = rb + M::row( lane, v );
-            const int     c0 = lane & 15, c1 = 16 + ( lane & 15 );
-            if ( rr < rows && c0 < bs ) base[rr * rs + c0 * ks] = M::get( acc0, v );
-            if ( rr < rows && c1 < bs ) base[rr * rs + c1 * ks] = M::get( acc1, v );
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// LU panel with static pivoting (core_zgetrfsp.c:64-272): the diagonal tile
-// of L holds the lower part of A_kk and the U tile its strict upper part,
-// transposed; they are summed (the reference's geadd), factorized without
-// pivoting by PXD_NB-column blocks (|a_kk| < tau -> sign(a_kk) tau), and the
-// packed LU is copied transposed into the U tile (the reference's getmo), so
-// that the lower part of the U tile is U^T.  The inverses of the diagonal
-// PXD_NB x PXD_NB blocks of L_kk (unit lower) and of U_kk^T go to the
-// diagonal blocks of DL and DU.
-template <typename T>
-__global__ void __launch_bounds__( PXD_THREADS )
-k_getrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__restrict__ L, T *__restrict__ U,
-          T *__restrict__ DL, T *__restrict__ DU, double thresh, int *__restrict__ npiv,
-          uint64_t *__restrict__ stamps, int prio )
-{
-    __shared__ T sA[PXD_NB][PXD_NB + 1];    // sA[col][row]
-    __shared__ T sIL[PXD_NB][PXD_NB + 1];   // L11^{-1}, [col][row]
-    __shared__ T sIU[PXD_NB][PXD_NB + 1];   // (U11^T)^{-1}, [col][row]
-    __shared__ T sD[PXD_NB];
-    __shared__ T sX[8][PXD_NB];              // exchange area of the elimination
-    __shared__ T sPi[PXD_NB][64 + 1];
-    __shared__ T sPj[PXD_NB][64 + 1];
-
-    const int32_t k   = list[blockIdx.x];
-    const uint64_t t_stamp = stamp_begin( stamps );
-    wave_priority( prio );
-    const dcblk   c   = cb[k];
-    const int32_t n   = c.lcolnum - c.fcolnum + 1;
-    const int     tid = threadIdx.x;
-    T *A  = L + c.coefoff;       // n x n, ld n
-    T *AU = U + c.coefoff;       // n x n, ld n
-    T *IL = DL + c.dinvoff;
-    T *IU = DU + c.dinvoff;
-    int     piv = 0;
-    typedef typename px_real<T>::type R;
-    const R tau = (R)thresh;
-    const int64_t nn = (int64_t)n * n;
-
-    // A_kk = L part + (U part)^T, 8 elements per thread in flight
-    for ( int64_t i0 = 0; i0 < nn; i0 += 8 * PXD_THREADS ) {
-        T va[8], vu[8];
-#pragma unroll
-        for ( int u = 0; u < 8; u++ ) {
-            const int64_t idx = i0 + tid + u * PXD_THREADS;
-            const int32_t r = (int32_t)( idx % n ), cc = (int32_t)( idx / n );
-            const bool    up = idx < nn && r < cc;
-            va[u] = up ? A[idx] : (T)0;
-            vu[u] = up ? AU[cc + (int64_t)r * n] : (T)0;
-        }
-#pragma unroll
-        for ( int u = 0; u < 8; u++ ) {
-            const int64_t idx = i0 + tid + u * PXD_THREADS;
-            const int32_t r = (int32_t)( idx % n ), cc = (int32_t)( idx / n );
-            if ( idx < nn && r < cc ) A[idx] = va[u] + vu[u];
-        }
-    }
-    __syncthreads();
-
-    for ( int32_t kb = 0; kb < n; kb += PXD_NB ) {
-        const int32_t bs = min( PXD_NB, n - kb );
-        {
-            constexpr int NU = PXD_NB * PXD_NB / PXD_THREADS;
-            T v[NU];
-#pragma unroll
-            for ( int u = 0; u < NU; u++ ) {
-                const int idx = tid + u * PXD_THREADS, r = idx % PXD_NB, cc = idx / PXD_NB;
-                v[u] = ( r < bs && cc < bs ) ? A[( kb + r ) + (int64_t)( kb + cc ) * n] : (T)0;
-            }
-#pragma unroll
-            for ( int u = 0; u < NU; u++ ) {
-                const int idx = tid + u * PXD_THREADS, r = idx % PXD_NB, cc = idx / PXD_NB;
-                sA[cc][r]  = v[u];
-                sIL[cc][r] = ( r == cc && r < bs ) ? (T)1 : (T)0;   // W_L = I
-                sIU[cc][r] = ( r == cc && r < bs ) ? (T)1 : (T)0;   // W_U = I
-            }
-        }
-        __syncthreads();
-
-        // unblocked right-looking LU, the multipliers left unscaled until the
-        // end; W_L = L11^{-1} and W_U = U~^{-1} (U11^T = U~ D, so that
-        // (U11^T)^{-1} = D^{-1} W_U) built alongside
-        piv += elim_lu32<T>( sA, sIL, sIU, sD, sX, bs, tau, tid );
-        for ( int idx = tid; idx < PXD_NB * PXD_NB; idx += PXD_THREADS ) {
-            const int rr = idx % PXD_NB, cc = idx / PXD_NB;
-            if ( rr >= bs || cc >= bs ) continue;
-            if ( rr > cc ) {
-                sA[cc][rr] = sA[cc][rr] / sD[cc];
-            }
-            else if ( rr == cc ) {
-                sA[cc][cc] = sD[cc];
-            }
-        }
-        __syncthreads();
-
-        // (U11^T)^{-1} = D^{-1} W_U: rows scaled by 1/d (W_L is L11^{-1} as is)
-        for ( int idx = tid; idx < PXD_NB * PXD_NB; idx += PXD_THREADS ) {
-            const int rr = idx % PXD_NB, cc = idx / PXD_NB;
-            if ( rr >= bs || cc >= bs ) continue;
-            if ( rr >= cc ) {
-                sIU[cc][rr] = sIU[cc][rr] / sD[rr];
-            }
-        }
-        __syncthreads();
-
-        for ( int idx = tid; idx < PXD_NB * PXD_NB; idx += PXD_THREADS ) {
-            const int rr = idx % PXD_NB, cc = idx / PXD_NB;
-            if ( rr >= bs || cc >= bs ) continue;
-            A[( kb + rr ) + (int64_t)( kb + cc ) * n]  = sA[cc][rr];
-            IL[( kb + rr ) + (int64_t)( kb + cc ) * n] = sIL[cc][rr];
-            IU[( kb + rr ) + (int64_t)( kb + cc ) * n] = sIU[cc][rr];
-        }
-
-        // in the tile: L21 <- A21 U11^{-1} = A21 (sIU)^T and
-        // U12^T <- A12^T L11^{-T} = A12^T (sIL)^T
-        const int32_t m0 = kb + bs;
-        const int32_t m  = n - m0;
-        small_trsm_mfma<T>( A + m0 + (int64_t)kb * n, 1, n, m, bs, sIU, tid );
-        small_trsm_mfma<T>( A + kb + (int64_t)m0 * n, n, 1, m, bs, sIL, tid );
-        __syncthreads();
-
-        // trailing update A22 -= L21 U12 (full square, 64 x 64 macro tiles)
-        const int32_t nt = ( m + 63 ) / 64;
-        const int     tx = tid % 16, ty = tid / 16;
-        for ( int32_t ti = 0; ti < nt; ti++ ) {
-            for ( int32_t tj = 0; tj < nt; tj++ ) {
-                {
-                    constexpr int NU = 64 * PXD_NB / PXD_THREADS;
-                    T vi[NU], vj[NU];
-#pragma unroll
-                    for ( int u = 0; u < NU; u++ ) {
-                        const int     idx = tid + u * PXD_THREADS, r = idx % 64, l = idx / 64;
-                        const int32_t ri = ti * 64 + r, rj = tj * 64 + r;
-                        vi[u] = ( ri < m && l < bs ) ? A[( m0 + ri ) + (int64_t)( kb + l ) * n] : (T)0;
-                        vj[u] = ( rj < m && l < bs ) ? A[( kb + l ) + (int64_t)( m0 + rj ) * n] : (T)0;
-                    }
-#pragma unroll
-                    for ( int u = 0; u < NU; u++ ) {
-                        const int idx = tid + u * PXD_THREADS, r = idx % 64, l = idx / 64;
-                        sPi[l][r] = vi[u];
-                        sPj[l][r] = vj[u];
-                    }
-                }
-                __syncthreads();
-                T acc[4][4];
-#pragma unroll
-                for ( int a = 0; a < 4; a++ )
-#pragma unroll
-                    for ( int b = 0; b < 4; b++ ) acc[a][b] = (T)0;
-                for ( int l = 0; l < bs; l++ ) {
-                    T ai[4], aj[4];
-#pragma unroll
-                    for ( int a = 0; a < 4; a++ ) {
-                        ai[a] = sPi[l][tx + 16 * a];
-                        aj[a] = sPj[l][ty + 16 * a];
-                    }
-#pragma unroll
-                    for ( int a = 0; a < 4; a++ )
-#pragma unroll
-                        for ( int b = 0; b < 4; b++ ) acc[a][b] += ai[a] * aj[b];
-                }
-                T old[4][4];
-#pragma unroll
-                for ( int a = 0; a < 4; a++ )
-#pragma unroll
-                    for ( int b = 0; b < 4; b++ ) {
-                        const int32_t r = ti * 64 + tx + 16 * a, cc = tj * 64 + ty + 16 * b;
-                        old[a][b] = ( r < m && cc < m ) ? A[( m0 + r ) + (int64_t)( m0 + cc ) * n] : (T)0;
-                    }
-#pragma unroll
-                for ( int a = 0; a < 4; a++ )
-#pragma unroll
-                    for ( int b = 0; b < 4; b++ ) {
-                        const int32_t r = ti * 64 + tx + 16 * a, cc = tj * 64 + ty + 16 * b;
-                        if ( r < m && cc < m ) A[( m0 + r ) + (int64_t)( m0 + cc ) * n] = old[a][b] - acc[a][b];
-                    }
-                __syncthreads();
-            }
-        }
-        __syncthreads();
-    }
-
-    // U tile <- (packed LU)^T, so that its lower part is U^T
-    for ( int64_t i0 = 0; i0 < nn; i0 += 8 * PXD_THREADS ) {
-        T va[8];
-#pragma unroll
-        for ( int u = 0; u < 8; u++ ) {
-            const int64_t idx = i0 + tid + u * PXD_THREADS;
-            va[u] = ( idx < nn ) ? A[idx] : (T)0;
-        }
-#pragma unroll
-        for ( int u = 0; u < 8; u++ ) {
-            const int64_t idx = i0 + tid + u * PXD_THREADS;
-            const int32_t r = (int32_t)( idx % n ), cc = (int32_t)( idx / n );
-            if ( idx < nn ) AU[cc + (int64_t)r * n] = va[u];
-        }
     }
     if ( tid == 0 && piv > 0 ) {
         atomicAdd( npiv, piv );
