@@ -26,6 +26,7 @@
 #include "kernels_solve.hpp"
 #include "kernels_mfma.hpp"
 #include "kernels_svsolve.hpp"
+#include "kernels_svwide.hpp"
 #include "kernels_panel.hpp"
 #include "pastix/kernels_enums.h"
 
@@ -43,6 +44,7 @@ struct level_t {
     int64_t f0, fs, f1; // solve row tasks (64-row tiles of off-diagonal rows); [fs, f1): Schur cblks
     int64_t d0, ds, d1; // solve diagonal tasks (PXD_DIAG_ROWS-row chunks of the diagonal blocks); [ds, d1): Schur
     int64_t m0, m1;     // one-wavefront solve tasks (levels whose cblks all fit one chunk, no Schur part)
+    int64_t w0, w1;     // backward blocks of the wide solve
     int64_t i0, i1;     // block-column inversion tasks
     int64_t g0, g1;     // blok updates (upd_group)
     int64_t q0, q1, q2; // panel tasks: [q0, q1) rows of the diagonal tiles, [q1, q2) columns of their inverses
@@ -125,12 +127,16 @@ struct pxd_ctx_s {
     sv_row   *dsvr  = nullptr;   // records of the off-diagonal stacked rows
     sv_chunk *dsvc  = nullptr;   // the diag tasks with their cblk sizes
     sv_small *dsvs  = nullptr;   // the one-wavefront solve tasks
+    sv_block *dsvb  = nullptr;   // the wide solve's backward blocks
     // backward partial sums of the cblks with many tiles (PXD_SV_SPREAD
     // copies of spread_cols columns x PXD_MAXRHS, factor precision)
     void     *dspread       = nullptr;
     size_t    dspread_bytes = 0;
     int64_t   spread_cols   = 0;
     int       solve_spread  = PXD_SV_SPREAD_MIN;   // fewest tiles of a cblk that spreads; 0: none
+    // fewest right-hand sides that a wide pass takes (kernels_svwide.hpp); 0:
+    // the rule of wide_from()
+    int       solve_wide_rhs = 0;
     // 1: levels of cblks of at most PXD_DIAG_ROWS columns solve with one
     // wavefront per cblk (diagonal and off-diagonal rows in one launch)
     int       solve_small = 1;
@@ -630,8 +636,32 @@ build_schedule( pxd_ctx_t *ctx )
             const int32_t n = c.lcolnum - c.fcolnum + 1;
             svs[i] = sv_small{ n, c.fcolnum, c.stride - n, 0, c.dinvoff, rowstart[smallk[i]] };
         }
+        // the wide solve's backward blocks: 64 to PXD_SVW_ROWS rows x 64
+        // columns, as many rows as leave the level PXD_SVW_BLOCKS of them
+        std::vector<sv_block> svb;
+        for ( int32_t lvl = 0; lvl < nlev; lvl++ ) {
+            level_t &lv = ctx->levels[lvl];
+            int64_t  nb = 0;
+            for ( int32_t k : bylev[lvl] ) {
+                const dcblk  &c = ctx->hcb[k];
+                const int32_t n = c.lcolnum - c.fcolnum + 1;
+                nb += (int64_t)( ( c.stride - n + 63 ) / 64 ) * ( ( n + 63 ) / 64 );
+            }
+            const int32_t step = 64 * (int32_t)std::max<int64_t>( 1, std::min<int64_t>( nb / PXD_SVW_BLOCKS, PXD_SVW_ROWS / 64 ) );
+            lv.w0 = svb.size();
+            for ( int32_t k : bylev[lvl] ) {
+                const dcblk  &c = ctx->hcb[k];
+                const int32_t n = c.lcolnum - c.fcolnum + 1, m = c.stride - n;
+                for ( int32_t r0 = 0; r0 < m; r0 += step ) {
+                    for ( int32_t c0 = 0; c0 < n; c0 += 64 ) {
+                        svb.push_back( sv_block{ n, c.fcolnum, c0, std::min( step, m - r0 ), rowstart[k] + r0 } );
+                    }
+                }
+            }
+            lv.w1 = svb.size();
+        }
         if ( upload( &ctx->dsvt, svt ) || upload( &ctx->dsvr, rows ) || upload( &ctx->dsvc, svc ) ||
-             upload( &ctx->dsvs, svs ) ) {
+             upload( &ctx->dsvs, svs ) || upload( &ctx->dsvb, svb ) ) {
             return 6;
         }
     }
@@ -1506,11 +1536,14 @@ graph_buffers( pxd_ctx_t *ctx )
     return 0;
 }
 
-// Both sweeps of nq columns held in ctx->dvecs, replayed from a graph that
-// is captured on first use (and again when what it baked in has changed).
-template <typename T>
+// Both sweeps of the columns held in ctx->dvecs (issued by `sweeps`), replayed
+// from a graph that is captured on first use (and again when what it baked in
+// has changed).  key: the columns of the pass, or those of a wide pass plus
+// PXD_WIDE_KEY.
+#define PXD_WIDE_KEY 1024
+template <typename T, typename F>
 int
-graph_pass( pxd_ctx_t *ctx, int nq )
+graph_pass( pxd_ctx_t *ctx, int nq, F sweeps )
 {
     const void *sig[7] = { ctx->dvecs, ctx->dsolvy, ctx->dL, ctx->dU, ctx->ddinv, ctx->dudinv,
                            ctx->solve_spread ? ctx->dspread : nullptr };
@@ -1532,7 +1565,7 @@ graph_pass( pxd_ctx_t *ctx, int nq )
         hipGraph_t     g  = nullptr;
         hipGraphExec_t ex = nullptr;
         PXD_CHECK( hipStreamBeginCapture( ctx->stream, hipStreamCaptureModeThreadLocal ) );
-        const int  rc = solve_sweeps<T, T>( ctx, (T *)ctx->dvecs, ctx->n, nq, SOLVE_ALL, false, nullptr );
+        const int  rc = sweeps();
         hipError_t e  = hipStreamEndCapture( ctx->stream, &g );
         if ( rc != 0 || e != hipSuccess || g == nullptr ) {
             if ( g ) (void)hipGraphDestroy( g );
@@ -1559,12 +1592,132 @@ graph_pass( pxd_ctx_t *ctx, int nq )
     return 0;
 }
 
+// Both sweeps of a wide pass (kernels_svwide.hpp): NR columns held by rows
+// in X, Y its second vector.
+template <typename T, int NR>
+int
+wide_sweeps( pxd_ctx_t *ctx, T *X, T *Y, int nq, bool swap )
+{
+    const bool  lu = ( ctx->facto == FACT_GETRF );
+    const T    *L  = (const T *)( swap ? ctx->dU : ctx->dL ), *DI = (const T *)( swap ? ctx->dudinv : ctx->ddinv );
+    const T    *LB = (const T *)( lu && !swap ? ctx->dU : ctx->dL );
+    const T    *DB = (const T *)( lu && !swap ? ctx->dudinv : ctx->ddinv );
+    hipStream_t s  = ctx->stream;
+    const dim3  th( PXD_THREADS );
+    auto        small = [&]( const level_t &lv ) { return ctx->solve_small && lv.m1 > lv.m0; };
+    for ( const level_t &lv : ctx->levels ) {
+        const unsigned nd = (unsigned)( lv.d1 - lv.d0 ), nf = (unsigned)( lv.f1 - lv.f0 );
+        if ( small( lv ) ) {
+            hipLaunchKernelGGL( ( k_svw_small_fwd<T, NR> ), dim3( (unsigned)( ( lv.m1 - lv.m0 + 3 ) / 4 ) ), th, 0, s,
+                                ctx->dsvs + lv.m0, lv.m1 - lv.m0, ctx->dsvr, L, DI, X, Y, nq );
+            continue;
+        }
+        if ( nd ) {
+            hipLaunchKernelGGL( ( k_svw_diag<T, NR> ), dim3( nd ), th, 0, s, ctx->dsvc + lv.d0, DI, (const T *)X, Y, 0 );
+        }
+        if ( nf ) {
+            int split = 1;
+            if ( (int64_t)nf < ctx->solve_wide_max ) {
+                split = std::max( 1, std::min( ctx->solve_split_max, (int)( ctx->solve_split_wg / (int64_t)nf ) ) );
+            }
+            hipLaunchKernelGGL( ( k_svw_fwd<T, NR> ), dim3( nf * split ), th, 0, s, ctx->dsvt + lv.f0, ctx->dsvr, L, X,
+                                (const T *)Y, nq, split );
+        }
+    }
+    if ( ctx->facto == FACT_SYTRF ) {
+        hipLaunchKernelGGL( ( k_svw_dscale<T, NR> ), dim3( nblocks( ctx->n * NR, 256 ) ), dim3( 256 ), 0, s,
+                            ctx->n, ctx->dcol2cblk, ctx->dcb, (const T *)ctx->dL, Y );
+    }
+    for ( int li = (int)ctx->levels.size() - 1; li >= 0; li-- ) {
+        const level_t &lv = ctx->levels[li];
+        const unsigned nd = (unsigned)( lv.d1 - lv.d0 ), nw = (unsigned)( lv.w1 - lv.w0 );
+        if ( small( lv ) ) {
+            hipLaunchKernelGGL( ( k_svw_small_bwd<T, NR> ), dim3( (unsigned)( ( lv.m1 - lv.m0 + 3 ) / 4 ) ), th, 0, s,
+                                ctx->dsvs + lv.m0, lv.m1 - lv.m0, ctx->dsvr, LB, DB, X, (const T *)Y );
+            continue;
+        }
+        if ( nw ) {
+            hipLaunchKernelGGL( ( k_svw_bwd<T, NR> ), dim3( nw ), th, 0, s, ctx->dsvb + lv.w0, ctx->dsvr, LB,
+                                (const T *)X, Y, nq );
+        }
+        if ( nd ) {
+            hipLaunchKernelGGL( ( k_svw_diag<T, NR> ), dim3( nd ), th, 0, s, ctx->dsvc + lv.d0, DB, (const T *)Y, X, 1 );
+        }
+    }
+    PXD_CHECK( hipGetLastError() );
+    return 0;
+}
+
+// One wide pass: nq <= NR columns of v.
+template <typename TV, typename T, int NR>
+int
+wide_pass( pxd_ctx_t *ctx, TV *v, int64_t ld, int nq, bool swap )
+{
+    const size_t need = (size_t)ctx->n * NR * sizeof( T );
+    if ( ctx->dvecs_bytes < need ) {
+        if ( ctx->dvecs ) PXD_CHECK( hipFree( ctx->dvecs ) );
+        ctx->dvecs       = nullptr;
+        ctx->dvecs_bytes = 0;
+        PXD_CHECK( hipMalloc( &ctx->dvecs, need ) );
+        ctx->dvecs_bytes = need;
+    }
+    if ( ctx->dsolvy_bytes < need ) {
+        if ( ctx->dsolvy ) PXD_CHECK( hipFree( ctx->dsolvy ) );
+        ctx->dsolvy       = nullptr;
+        ctx->dsolvy_bytes = 0;
+        PXD_CHECK( hipMalloc( &ctx->dsolvy, need ) );
+        ctx->dsolvy_bytes = need;
+    }
+    T   *X = (T *)ctx->dvecs, *Y = (T *)ctx->dsolvy;
+    auto sweeps = [&] { return wide_sweeps<T, NR>( ctx, X, Y, nq, swap ); };
+    hipLaunchKernelGGL( ( k_svw_pack<T, TV, NR> ), dim3( nblocks( ctx->n, 64 ) ), dim3( PXD_THREADS ), 0, ctx->stream,
+                        ctx->n, (const TV *)v, ld, nq, X );
+    const int rc = graph_ok( ctx, SOLVE_ALL, swap ) ? graph_pass<T>( ctx, PXD_WIDE_KEY + nq, sweeps ) : sweeps();
+    hipLaunchKernelGGL( ( k_svw_unpack<T, TV, NR> ), dim3( nblocks( ctx->n, 64 ) ), dim3( PXD_THREADS ), 0, ctx->stream,
+                        ctx->n, (const T *)X, nq, v, ld );
+    return rc;
+}
+
+// Fewest right-hand sides for which a wide pass is the faster one (measured,
+// narrow against wide): in double always (100^3: 5.80 against 5.22 ms for 1
+// and 9.7 against 5.8 ms for 8; 41^3 LU 0.59 / 0.51 ms for 1); in single from
+// 5 on (100^3: 4.14 against 4.92 ms for 4, 5.48 against 4.80 ms for 5), and on
+// small systems, which are all latency, always (25^3: 0.23 against 0.16 ms
+// for 4; 50^3, 125,000 unknowns: 0.698 against 0.701 ms).
+template <typename T>
+int64_t
+wide_from( const pxd_ctx_t *ctx )
+{
+    if ( ctx->solve_wide_rhs > 0 ) {
+        return ctx->solve_wide_rhs;
+    }
+    return sizeof( typename px_real<T>::type ) == 8 || ctx->n < 100000 ? 1 : 5;
+}
+
 template <typename TV, typename T>
 int
 solve_vectors( pxd_ctx_t *ctx, int64_t nrhs, void *dx, int64_t ldx, int what = SOLVE_ALL, bool swap = false,
                void *scr = nullptr )
 {
     int rc = 0;
+    // Wide passes of 32, 16 and 4 columns where they are the faster ones, the
+    // rest by the narrow ones below, which also keep the sweeps on their own,
+    // the Schur parts, the scalar kernels and the allocation-free solve.
+    if ( scr == nullptr && what == SOLVE_ALL && ctx->kernels && ctx->schurfcol >= ctx->n ) {
+        TV *v = (TV *)dx;
+        while ( nrhs > 0 && nrhs >= wide_from<T>( ctx ) && rc == 0 ) {
+            const int nq = (int)std::min<int64_t>( nrhs, 32 );
+            rc = nq > 16  ? wide_pass<TV, T, 32>( ctx, v, ldx, nq, swap )
+                 : nq > 4 ? wide_pass<TV, T, 16>( ctx, v, ldx, nq, swap )
+                          : wide_pass<TV, T, 4>( ctx, v, ldx, nq, swap );
+            v += nq * ldx;
+            nrhs -= nq;
+        }
+        if ( rc != 0 || nrhs == 0 ) {
+            return rc;
+        }
+        dx = v;
+    }
     const bool graph = scr == nullptr && graph_ok( ctx, what, swap );
     if ( graph && ( rc = graph_buffers<T>( ctx ) ) != 0 ) {
         return rc;
@@ -1578,7 +1731,7 @@ solve_vectors( pxd_ctx_t *ctx, int64_t nrhs, void *dx, int64_t ldx, int what = S
                 T *xs = (T *)ctx->dvecs;
                 hipLaunchKernelGGL( ( k_copy_cols<T> ), dim3( nblocks( ctx->n, 256 ), nq ), dim3( 256 ), 0,
                                     ctx->stream, ctx->n, (const T *)dx + q0 * ldx, ldx, xs, ctx->n );
-                rc = graph_pass<T>( ctx, nq );
+                rc = graph_pass<T>( ctx, nq, [&] { return solve_sweeps<T, T>( ctx, xs, ctx->n, nq ); } );
                 hipLaunchKernelGGL( ( k_copy_cols<T> ), dim3( nblocks( ctx->n, 256 ), nq ), dim3( 256 ), 0,
                                     ctx->stream, ctx->n, (const T *)xs, ctx->n, (T *)dx + q0 * ldx, ldx );
             }
@@ -1612,7 +1765,8 @@ solve_vectors( pxd_ctx_t *ctx, int64_t nrhs, void *dx, int64_t ldx, int what = S
                 hipLaunchKernelGGL( ( k_convert<T, TV> ), dim3( nblocks( ctx->n, 256 ) ), dim3( 256 ), 0, ctx->stream,
                                     ctx->n, (const TV *)dx + ( q0 + q ) * ldx, xs + q * ctx->n );
             }
-            rc = graph ? graph_pass<T>( ctx, nq ) : solve_sweeps<T, T>( ctx, xs, ctx->n, nq, what, swap, ys );
+            rc = graph ? graph_pass<T>( ctx, nq, [&] { return solve_sweeps<T, T>( ctx, xs, ctx->n, nq ); } )
+                       : solve_sweeps<T, T>( ctx, xs, ctx->n, nq, what, swap, ys );
             for ( int q = 0; q < nq; q++ ) {
                 hipLaunchKernelGGL( ( k_convert<TV, T> ), dim3( nblocks( ctx->n, 256 ) ), dim3( 256 ), 0, ctx->stream,
                                     ctx->n, xs + q * ctx->n, (TV *)dx + ( q0 + q ) * ldx );
@@ -1853,7 +2007,7 @@ pxd_destroy( pxd_ctx_t *ctx )
     if ( ctx->fgraph ) {
         (void)hipGraphExecDestroy( ctx->fgraph );
     }
-    void *ptrs[] = { ctx->dcb, ctx->dbk, ctx->dcol2cblk, ctx->dlist, ctx->dpan, ctx->dflags, ctx->dtrsm, ctx->dupd, ctx->dupdb, ctx->dupds, ctx->dsolv, ctx->dsvt, ctx->dsvr, ctx->dsvc, ctx->dsvs, ctx->dspread, ctx->ddiag, ctx->dsolvy, ctx->dinvt,
+    void *ptrs[] = { ctx->dcb, ctx->dbk, ctx->dcol2cblk, ctx->dlist, ctx->dpan, ctx->dflags, ctx->dtrsm, ctx->dupd, ctx->dupdb, ctx->dupds, ctx->dsolv, ctx->dsvt, ctx->dsvr, ctx->dsvc, ctx->dsvs, ctx->dsvb, ctx->dspread, ctx->ddiag, ctx->dsolvy, ctx->dinvt,
                      ctx->dcolptr, ctx->drowtab, ctx->dtcolptr, ctx->dtrowtab, ctx->dval, ctx->dtval,
                      ctx->dL, ctx->dU, ctx->ddinv, ctx->dudinv, ctx->dscratch, ctx->dvecs, ctx->dred,
                      };
@@ -1918,6 +2072,13 @@ pxd_set_option( pxd_ctx_t *ctx, const char *key, double value )
     if ( k == "solve_small" ) {
         ctx->solve_small = ( value != 0. );
         drop_solve_graphs( ctx );
+        return 0;
+    }
+    if ( k == "solve_wide_rhs" ) {
+        if ( value < 1. || value > 1e9 ) {
+            return 7;
+        }
+        ctx->solve_wide_rhs = (int)value;
         return 0;
     }
     if ( k == "solve_split_max" || k == "solve_split_wg" ) {

@@ -1,0 +1,58 @@
+"""The passes of 16 and 32 right-hand sides against the narrow passes of at
+most 8 (option solve_wide_rhs) on the same factor: the same sums in another
+order, so they agree to rounding of the factor precision.  Counts at the
+edges of the passes, every factorization and arithmetic, LU's transposed
+solve, leaf levels on the one-wavefront kernels and on the tiles
+(solve_small), eager and replayed from graphs, and cblks of one to five
+64-column blocks with rows that end inside a 64-row step."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import pastix_amd as px
+from helpers import analyzed, make_problem
+
+pytestmark = pytest.mark.gpu
+
+CASES = [("lap7", px.PastixFactPOTRF, 0, (13, 17, 18)), ("lap7", px.PastixFactPOTRF, 1, (13, 17, 18)),
+         ("lap7sd", px.PastixFactLDLT, 0, (9, 10, 11)), ("vlap7", px.PastixFactLDLT, 1, (9, 10, 11)),
+         ("convdiff27", px.PastixFactLU, 0, (11, 9, 10)), ("convdiff27", px.PastixFactLU, 1, (11, 9, 10)),
+         ("helmholtz7", px.PastixFactLDLT, 0, (10, 11, 9)), ("helmholtz7", px.PastixFactLDLT, 1, (10, 11, 9)),
+         ("helmholtz7", px.PastixFactLU, 0, (8, 9, 9)), ("helmholtz7", px.PastixFactLU, 1, (8, 9, 9))]
+
+
+def _solve(pd, b, trans):
+    n, nrhs = b.shape
+    dev, dx = ctypes.c_void_p(), ctypes.c_void_p()
+    px._check("device", px.lib.pastix_amd_device_handle(pd, ctypes.byref(dev)))
+    x = np.array(b, order="F", copy=True)
+    px._check("malloc", px.lib.pxd_malloc(dev, x.nbytes, ctypes.byref(dx)))
+    px.lib.pxd_h2d(dev, dx, x.ctypes.data_as(ctypes.c_void_p), x.nbytes)
+    f = px.lib.pxd_solve_trans
+    f.argtypes = [ctypes.c_void_p, ctypes.c_int, px.pastix_int, ctypes.c_void_p, px.pastix_int]
+    px._check("pxd_solve_trans", f(dev, int(trans), nrhs, dx, n))
+    px.lib.pxd_d2h(dev, x.ctypes.data_as(ctypes.c_void_p), dx, x.nbytes)
+    px.lib.pxd_free(dev, dx)
+    return x
+
+
+@pytest.mark.parametrize("kind,facto,mixed,edges", CASES)
+def test_wide_passes_match_narrow_passes(kind, facto, mixed, edges):
+    spm = make_problem(kind, *edges, dof=1)
+    pd, iparm, dparm = analyzed(spm, *edges, facto=facto, mixed=mixed)
+    px.task_numfact(pd, spm)
+    eps = np.finfo(np.float32 if mixed else np.float64).eps
+    for nrhs, trans, small, graph in [(1, 0, 1, 1), (5, 0, 1, 1), (16, 0, 1, 1), (17, 0, 0, 1), (32, 0, 1, 0),
+                                      (33, 0, 1, 1), (33, 0, 1, 1), (49, 1, 1, 1), (20, 1, 0, 0)]:
+        px.set_option(pd, "solve_small", small)
+        px.set_option(pd, "solve_graph", graph)
+        _, b = spm.gen_rhs(nrhs, seed=nrhs)
+        px.set_option(pd, "solve_wide_rhs", 1e9)
+        want = _solve(pd, b, trans)
+        px.set_option(pd, "solve_wide_rhs", 1)
+        got = _solve(pd, b, trans)
+        assert np.abs(got - want).max() <= 200 * eps * np.abs(want).max(), (nrhs, trans, small, graph)
+    with pytest.raises(px.PastixError):
+        px.set_option(pd, "solve_wide_rhs", 0)
+    px.finalize(pd)
