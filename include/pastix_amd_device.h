@@ -91,11 +91,10 @@ int  pxd_get_stats( const pxd_ctx_t *ctx, pxd_stats_t *stats );
  *                   64) and facing columns (up to 64, default 16) of an
  *                   update that goes to the one-wavefront kernel (one
  *                   wavefront per 64 rows; at most 32 source columns)
- *   "upd_dma"       1: single-precision LL^T / LU tall tiles load their
- *                   operands straight into LDS (default); 0: register-staged
- *   "upd_dma_pad"   extra LDS bytes per workgroup of that kernel (0..65536,
- *                   default 4096: four workgroups per CU, room left for the
- *                   lookahead stream's panels)
+ *   "upd_dma"       1: tall update tiles load their operands straight into
+ *                   LDS (default); 0: through registers
+ *   "upd_dma_pad"   extra LDS bytes per single-precision workgroup of that
+ *                   kernel (0..65536, default 4096)
  *   "fact_graph"    1: the factorization's level loop replays a graph
  *                   captured once per structure (default)
  *   "prio"          1: raised wave priority on the critical path (default)

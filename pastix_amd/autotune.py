@@ -14,8 +14,8 @@ rounding:
 - ``solve_wide_max``: level-solve launches from which the tiles load 16
   columns per batch instead of all of them;
 - ``panel_mw``: the multi-workgroup Cholesky panel;
-- ``upd_dma``: single-precision tall tiles on the kernel that loads its
-  operands straight into LDS;
+- ``upd_dma``: tall tiles on the kernel that loads its operands straight
+  into LDS;
 - ``upd_dma_pad``: extra LDS per workgroup of that kernel, which sets how
   many of its workgroups share a CU with the lookahead stream's panels;
 - ``solve_split_max``, ``solve_split_wg``: how many workgroups share a tile

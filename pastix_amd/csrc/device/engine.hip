@@ -193,17 +193,16 @@ struct pxd_ctx_s {
     int          upd_small_n = 16;
     // stacked rows per tall tile (upd_rows<T>, set with the factor precision)
     int          upd_bm = 256;
-    // 1: single-precision LL^T / LU tall tiles on the kernel that loads its
-    // operands straight into LDS (k_update_dma); 0: on k_update_big
+    // 1: tall tiles on the kernel that loads its operands straight into LDS
+    // (k_update_dma); 0: on k_update_big
     int          upd_dma = 1;
     // level-solve launches with fewer than solve_wide_max tiles share each
     // tile among up to solve_split_max workgroups, solve_split_wg in all
     int          solve_split_max = 4;
     int64_t      solve_split_wg  = 512;
-    // dynamic LDS bytes added to each k_update_dma workgroup: 4 KiB makes it
-    // 34 KiB, four workgroups per CU, and leaves 24 KiB of the CU's LDS to the
-    // panel and TRSM workgroups of the lookahead stream (without it, or with
-    // less free, the next level's panels wait for a CU)
+    // dynamic LDS bytes added to each single-precision k_update_dma workgroup:
+    // up to 8 KiB there are four per CU, with room for the panel workgroups of
+    // the lookahead stream
     unsigned     upd_dma_pad = 4096;
 
     // host copies of the panel, TRSM and inversion lists, and the blok
@@ -998,16 +997,18 @@ factorize( pxd_ctx_t *ctx, double thresh, int64_t *nbpivots )
             launches++;
         }
         if ( nb ) {
-            bool done = false;
-            if constexpr ( std::is_same<T, float>::value ) {
-                if ( ctx->upd_dma && !ldlt ) {
-                    hipLaunchKernelGGL( ( k_update_dma<PXD_DMA_BK, PXD_DMA_NBUF> ), dim3( nb ), dim3( PXD_THREADS ),
-                                        ctx->upd_dma_pad, st, ctx->dupdb + b0, (int32_t)nb, ctx->dcb, ctx->dbk, L, U,
-                                        stp( st_updb, b0, 0, 0 ), prio );
-                    done = true;
-                }
+            const unsigned pad = dma_shape<T>::pad < 0 ? ctx->upd_dma_pad : (unsigned)dma_shape<T>::pad;
+            if ( ctx->upd_dma && ldlt ) {
+                hipLaunchKernelGGL( ( k_update_dma<T, true> ), dim3( nb ), dim3( PXD_THREADS ), pad, st,
+                                    ctx->dupdb + b0, (int32_t)nb, ctx->dcb, ctx->dbk, L, U, stp( st_updb, b0, 0, 0 ),
+                                    prio );
             }
-            if ( !done ) {
+            else if ( ctx->upd_dma ) {
+                hipLaunchKernelGGL( ( k_update_dma<T, false> ), dim3( nb ), dim3( PXD_THREADS ), pad, st,
+                                    ctx->dupdb + b0, (int32_t)nb, ctx->dcb, ctx->dbk, L, U, stp( st_updb, b0, 0, 0 ),
+                                    prio );
+            }
+            else {
                 hipLaunchKernelGGL( ( k_update_big<T, 1> ), dim3( nb ), dim3( PXD_THREADS ), 0, st, ctx->dupdb + b0,
                                     (int32_t)nb, ctx->dcb, ctx->dbk, L, U, ldlt, stp( st_updb, b0, 0, 0 ), prio );
             }

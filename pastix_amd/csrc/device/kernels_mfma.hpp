@@ -1467,62 +1467,118 @@ k_update_big( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
 
 
 // ---------------------------------------------------------------------------
-// Single-precision tall-tile update (the 256 x 64 tiles of k_update_big<float>,
-// real LL^T and LU) with its operands moved from HBM straight into LDS by
-// buffer loads that write LDS (no register staging), in a ring of NBUF
-// buffers of BK k values: while a stage's products run, the loads of the
-// next NBUF - 1 stages are in flight, and each stage ends with one barrier.  The staged tiles are k
-// major (sA[k][256 rows], sB[k][64 columns]), so a load instruction moves one
-// k value of 64 consecutive rows (one wave) and every lane writes LDS at its
-// own consecutive word.  A 16-byte LDS read then gives a lane one k value of
-// four rows (or columns): the wave's 64 x 64 block is cut into 16 x 16
-// matrix-core tiles by interleaving, tile i (j) taking the rows (columns)
-// 4 r + i of the block, so that the four values of one read feed the four
-// row (column) tiles of one k step.  The scatter into the facing cblk is the
-// one of k_update_big: a 16-column slab at a time, transposed through LDS so
-// that a lane owns one row and each memory instruction covers 64 consecutive
-// rows of one column.
+// Tall-tile update with its operands moved from HBM straight into LDS by
+// buffer loads that write LDS (no register staging), in a ring of NBUF buffers
+// of BK k values: while a stage's products run, the loads of the next NBUF - 1
+// stages are in flight, and each stage ends with one barrier.
 //
-// The row mapped by thread tid is row tid of the tile, for the loads and for
-// the scatter alike, so its offsets stay in registers.  The LDS holds the
-// ring and nothing else (NBUF x BK x 1280 bytes); the search keys live in the
-// last buffer until its first load, and the scatter's transposes in the A
-// buffers after the last stage.
-#define PXD_DMA_BM 256
-// measured on the 100^3 FP32 factorization: 8 k values in a ring of 3 (loads
-// of the next two stages in flight, 30 KiB) ahead of 16 x 2 (40 KiB), 12 x 2,
-// 12 x 3 and 8 x 4
-#define PXD_DMA_BK   8
-#define PXD_DMA_NBUF 3
-template <int BK, int NBUF>
+// The staged tiles are k major (A[k][BM rows], B[k][64 columns]).  A load
+// instruction moves 64 dwords (one k value of 64 rows of float, of 32 rows of
+// the 8-byte types, whose two dwords go to a lane pair) or 64 elements of 16
+// bytes; every lane writes LDS at its own consecutive place.  Wave w computes
+// the rows [w BM/4, (w+1) BM/4) of the tile and, except in complex double,
+// loads the same ones.
+//
+// C -= acc goes a 16-column slab at a time through LDS, each wave for itself,
+// so that a memory instruction covers the wave's 16 to 64 consecutive rows of
+// one column.  The runs matter more than the barriers: straight from the
+// accumulators (runs of 16 rows) the 100^3 float updates took 73.6 ms, by
+// slabs 65.3 ms.  The rows' places in the facing cblk are in the registers of
+// the lanes that loaded them.
+//
+// What bounds it: the read-modify-write of C beside the products.  100^3,
+// update launches alone: float 66.7 -> 65.3 ms against the same scheme with
+// two workgroup barriers per slab and no load in flight across a stage's
+// barrier, double 136.2 -> 133.2 ms and 80^3 complex64 LDL^T 73.0 -> 71.8 ms
+// against k_update_big (factorizations 155.8 -> 150.7 and 88.0 -> 84.9 ms).
+//
+// LDL^T scales A by D (kept in LDS), the reference's D L^T workspace.
+
+// 4 or 16 bytes per lane from r + off to LDS, at the lane's place from dst on
+template <int BYTES>
+__device__ inline void
+load_lds( __amdgpu_buffer_rsrc_t r, void *dst, uint32_t off )
+{
+    typedef __attribute__( ( address_space( 3 ) ) ) void lds_t;
+    if constexpr ( BYTES == 16 ) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds( r, (lds_t *)dst, 16, off, 0, 0, 0 );
+    }
+    else {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds( r, (lds_t *)dst, 4, off, 0, 0, 0 );
+    }
+}
+// Barrier of the workgroup alone: no wait for memory, and no memory access of
+// the wave moves across it (wavefront fences order the compiler only).
+__device__ inline void
+bare_barrier()
+{
+    __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
+}
+// k values per stage, and dynamic LDS that leaves CU room to the panels of the
+// other stream (float: option upd_dma_pad; complex double 19.1 -> 18.3 ms at
+// 50^3 with three workgroups per CU instead of four; in double and complex
+// float fewer than four cost more than they give: 150.7 -> 155.6 and 84.9 ->
+// 86.9 ms)
+template <typename T> struct dma_shape;
+template <> struct dma_shape<float>  { static constexpr int bk = 8, pad = -1; };
+template <> struct dma_shape<double> { static constexpr int bk = 8, pad = 0; };
+template <> struct dma_shape<pxcf>   { static constexpr int bk = 8, pad = 0; };
+template <> struct dma_shape<pxcd>   { static constexpr int bk = 4, pad = 10240; };
+
+template <typename T, bool LDLT>
 __global__ void __launch_bounds__( PXD_THREADS, 4 )
 k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *__restrict__ cb,
-              const dblok *__restrict__ bk, float *L, float *U, uint64_t *__restrict__ stamps, int prio )
+              const dblok *__restrict__ bk, T *L, T *U, uint64_t *__restrict__ stamps, int prio )
 {
-    typedef mfma16<float> M;
-    typedef M::acc_t      acc_t;
-    typedef float f4 __attribute__( ( ext_vector_type( 4 ) ) );
-    constexpr int      BM = PXD_DMA_BM, BN = PXD_UPD_BN;
-    constexpr uint32_t ES = sizeof( float );
-    static_assert( BK % 4 == 0, "a stage is a whole number of 4-k matrix-core steps (one per wave for B)" );
-    static_assert( NBUF >= 2 && NBUF <= 4, "ring of 2 to 4 stages" );
-    static_assert( PXD_THREADS == BM, "thread tid maps row tid of the tile" );
-    static_assert( upd_rows<float>::value == BM, "the tall-tile list of a single factor has 256-row tiles" );
-    static_assert( sizeof( search_keys ) <= BK * BM * sizeof( float ), "search keys fit in one A buffer" );
-    static_assert( 4 * 64 * 17 <= NBUF * BK * BM, "scatter transposes fit in the A buffers" );
-    constexpr int LPS = BK + BK / 4;                    // loads per stage and wave
-    constexpr int VMN = LPS * ( NBUF - 2 );             // loads issued after the next stage's
+    typedef mfma16<T>         M;
+    typedef typename M::acc_t acc_t;
+    constexpr int      BK = dma_shape<T>::bk, NBUF = 3;
+    constexpr int      BM = upd_rows<T>::value, BN = PXD_UPD_BN;
+    constexpr uint32_t ES = sizeof( T );
+    constexpr int      LPE = ( ES == 8 ) ? 2 : 1;            // lanes per element of a load
+    constexpr int      LSZ = ( ES == 16 ) ? 16 : 4;          // bytes per lane of a load
+    constexpr int      RPI = 64 / LPE;                       // rows (columns of B) per load
+    constexpr int      WR  = BM / 4, RB = WR / 16;           // rows and 16-row blocks per wave
+    constexpr bool     OWN = ( RPI == WR );                  // a wave loads its own rows (else all rows of its k)
+    constexpr int      QA  = OWN ? BK : BK / 4;              // loads per stage and wave
+    constexpr int      QB  = BK * BN / RPI / 4;
+    constexpr int      BG  = BN / RPI;                       // loads per k value of B
+    constexpr int      AST = BM + ( ES == 4 ? 16 : 0 );      // float: k values 64 bytes apart, else two meet in a bank
+    constexpr int      LPS = QA + QB;
+    constexpr int      VMN = LPS * ( NBUF - 2 );             // loads issued after the next stage's
+    static_assert( BK % 4 == 0, "stages of whole 4-k products" );
+    static_assert( OWN || RPI == BM, "a load covers a wave's rows or the whole tile's" );
     static_assert( VMN < 64, "vmcnt holds 6 bits" );
+    static_assert( sizeof( search_keys ) <= BK * AST * ES, "search keys fit in one A buffer" );
     constexpr int WAIT_NEXT = ( VMN & 15 ) | ( ( VMN >> 4 ) << 14 ) | 0x0F70;   // s_waitcnt vmcnt(VMN)
-    __shared__ __align__( 16 ) float smem[NBUF * BK * ( BM + BN )];
-    search_keys &sk = *reinterpret_cast<search_keys *>( smem + ( NBUF - 1 ) * BK * BM );
+    constexpr int DN = PXD_TRSM_NT * 16 + BK;
+    // one variable per stage (A, then B): the compiler tells loads into one
+    // from reads of another only by the variable, and waits for all of them
+    // where it cannot
+    __shared__ __align__( 16 ) T stage0[BK * ( AST + BN )];
+    __shared__ __align__( 16 ) T stage1[BK * ( AST + BN )];
+    __shared__ __align__( 16 ) T stage2[BK * ( AST + BN )];
+    T *sD = nullptr;
+    if constexpr ( LDLT ) {
+        __shared__ T sDk[DN];
+        sD = sDk;
+    }
+    auto buffer = [&]( auto bc ) -> T * {
+        constexpr int b = decltype( bc )::value;
+        if constexpr ( b == 0 ) return stage0;
+        else if constexpr ( b == 1 ) return stage1;
+        else return stage2;
+    };
+    search_keys &sk = *reinterpret_cast<search_keys *>( stage2 );
 
     const int32_t  ti      = xcd_task( blockIdx.x, ntasks );
     const upd_task t       = tasks[ti];
     const uint64_t t_stamp = stamp_begin( stamps );
     wave_priority( prio );
     const int     tid = threadIdx.x;
-    const int     lane = tid & 63, w = tid >> 6;
+    const int     lane = tid & 63, w = __builtin_amdgcn_readfirstlane( tid >> 6 );
     const dcblk   c   = cb[t.cblk];
     const int32_t K   = c.lcolnum - c.fcolnum + 1;
     const int32_t lb  = cb[t.cblk + 1].fblok;
@@ -1530,9 +1586,9 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
     const int32_t N   = bb.lrownum - bb.frownum + 1;
     // U-side tile (LU): A = U^T rows after blok b, B = L rows of blok b, C = U
     const bool    uside = ( t.flags & 2 ) != 0;
-    const float  *LA    = uside ? U : L;
-    const float  *LB    = uside ? L : U;
-    float        *LC    = uside ? U : L;
+    const T      *LA    = uside ? U : L;
+    const T      *LB    = uside ? L : U;
+    T            *LC    = uside ? U : L;
     const int32_t r0    = bb.rowoff + ( uside ? N : 0 );
     const int32_t Mr    = c.stride - r0;
     const int32_t F     = bb.fcblknm;
@@ -1548,18 +1604,23 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
     const __amdgpu_buffer_rsrc_t rC = make_rsrc( LC + cf.coefoff, (uint32_t)( (int64_t)cf.stride * Fn * ES ) );
 
     stage_search_keys( sk, bk, t.blok, lb, cf.fblok, flb, tid );
+    if constexpr ( LDLT ) {
+        for ( int32_t i = tid; i < DN; i += PXD_THREADS ) {
+            sD[i] = ( i < K ) ? L[c.coefoff + (int64_t)i * ( K + 1 )] : (T)0;
+        }
+    }
     __syncthreads();
 
-    // row tid of the tile: byte offset of its first element and byte stride
-    // between its columns in the source, and its place in F
+    // the lane's row of the tile: byte offset of its part of the first element
+    // and byte stride between its columns in the source, and its place in F
     uint32_t abase = PXD_OOB, astep = 0, dst = PXD_OOB, dld = 0;
     {
-        const int32_t r = t.tm * BM + tid;
+        const int32_t r = t.tm * BM + ( OWN ? WR * w : 0 ) + lane / LPE;
         if ( r < Mr ) {
             const int32_t s  = r0 + r;
             const dblok   ib = bk[search_row( sk, bk, t.blok, lb, s )];
             const int32_t g  = ib.frownum + ( s - ib.rowoff );
-            abase = (uint32_t)( ib.rowoff * K + ( s - ib.rowoff ) ) * ES;
+            abase = (uint32_t)( ib.rowoff * K + ( s - ib.rowoff ) ) * ES + LSZ * ( lane % LPE );
             astep = (uint32_t)( ib.lrownum - ib.frownum + 1 ) * ES;
             const dblok fb = bk[search_grow( sk, bk, cf.fblok, flb, g )];
             if ( g >= fb.frownum && g <= fb.lrownum ) {
@@ -1568,44 +1629,64 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
             }
         }
     }
-    // facing column `lane` of the tile
+    // the lane's facing column: wave w loads the columns of group w % BG at
+    // the k values w / BG, w / BG + 4 / BG, ... of a stage
+    constexpr int  KSB    = 4 / BG;
     const int32_t  nvalid = min( BN, N - t.tn * BN );
-    const uint32_t bbase  = ( lane < nvalid ) ? (uint32_t)( bb.rowoff * K + t.tn * BN + lane ) * ES : PXD_OOB;
-    const uint32_t bstep  = ( lane < nvalid ) ? (uint32_t)N * ES : 0;
+    const int      bcol   = RPI * ( w % BG ) + lane / LPE, bk0 = w / BG;
+    uint32_t       bo = PXD_OOB, bstep = 0;
+    if ( bcol < nvalid ) {
+        bo    = (uint32_t)( bb.rowoff * K + t.tn * BN + bcol ) * ES + LSZ * ( lane % LPE ) + (uint32_t)( bk0 * N ) * ES;
+        bstep = (uint32_t)( KSB * N ) * ES;
+    }
+    const int ak0 = OWN ? 0 : w;
+    uint32_t  ao = ( abase == PXD_OOB ) ? PXD_OOB : abase + (uint32_t)ak0 * astep;
+    if constexpr ( !OWN ) astep *= 4;
 
-    // stage k0 into buffer b: wave w loads the BK k values of rows
-    // [64 w, 64 w + 64) and k values w, w + 4, ... of the 64 columns.  The
-    // offsets advance by one column per load (ao, bo carried from stage to
-    // stage), so that no per-k products stay live across the loop.
-    const int wu = __builtin_amdgcn_readfirstlane( w );
-    uint32_t  ao = abase, bo = ( bbase == PXD_OOB ) ? PXD_OOB : bbase + (uint32_t)wu * bstep;
+    // stage k0 into buffer b; the offsets advance from load to load, so that
+    // no per-k products stay live across the loop
     auto dma = [&]( auto bc, int32_t k0 ) {
-        constexpr int b  = decltype( bc )::value;
-        float        *dA = smem + b * ( BK * BM ) + 64 * wu;
-        float        *dB = smem + NBUF * BK * BM + b * ( BK * BN ) + wu * BN;
+        T            *dA = buffer( bc ) + ( OWN ? WR * w : w * AST );
+        T            *dB = buffer( bc ) + BK * AST + bk0 * BN + RPI * ( w % BG );
         const bool    full = ( k0 + BK <= K );
 #pragma unroll
-        for ( int q = 0; q < BK; q++ ) {
-            const uint32_t o = ( full || k0 + q < K ) ? ao : PXD_OOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds( rA, (__attribute__( ( address_space( 3 ) ) ) void *)( dA + q * BM ),
-                                                      4, o, 0, 0, 0 );
+        for ( int q = 0; q < QA; q++ ) {
+            constexpr int  KSA = OWN ? 1 : 4;
+            const uint32_t o = ( full || k0 + KSA * q + ak0 < K ) ? ao : PXD_OOB;
+            load_lds<LSZ>( rA, dA + KSA * q * AST, o );
             ao += astep;
         }
 #pragma unroll
-        for ( int q = 0; q < BK / 4; q++ ) {
-            const uint32_t o = ( full || k0 + 4 * q + wu < K ) ? bo : PXD_OOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rB, (__attribute__( ( address_space( 3 ) ) ) void *)( dB + 4 * q * BN ), 4, o, 0, 0, 0 );
-            bo += 4 * bstep;
+        for ( int q = 0; q < QB; q++ ) {
+            const uint32_t o = ( full || k0 + KSB * q + bk0 < K ) ? bo : PXD_OOB;
+            load_lds<LSZ>( rB, dB + KSB * q * BN, o );
+            bo += bstep;
         }
     };
 
-    acc_t acc[4][4];
+    acc_t acc[RB][4];
 #pragma unroll
-    for ( int i = 0; i < 4; i++ )
+    for ( int i = 0; i < RB; i++ )
 #pragma unroll
         for ( int j = 0; j < 4; j++ ) acc[i][j] = M::zero();
 
+    // End of a stage: this wave's loads of the next stage are in LDS (those of
+    // the one after, issued since, may be in flight), and after the barrier
+    // every wave's are.  The products stay ahead of it, so every LDS read of
+    // the stage has returned.  Not __syncthreads(): its fence waits for the
+    // loads in flight too (vmcnt 0), which leaves no stage ahead of the
+    // products.
+    auto next_stage = []() {
+        __builtin_amdgcn_sched_barrier( 0 );
+        __builtin_amdgcn_s_waitcnt( WAIT_NEXT );
+        bare_barrier();
+        __builtin_amdgcn_sched_barrier( 0 );
+    };
+
+    // 16-byte reads of B: VB columns next to each other feed VB of the four
+    // column tiles (tile j holds the columns 16 VB (j / VB) + VB r + j % VB)
+    constexpr int VB = 16 / ES;
+    struct __align__( 16 ) bvec { T e[VB]; };
     const int     lr = lane & 15, lg = lane >> 4;
     const int32_t ns = ( K + BK - 1 ) / BK;
     // stage s from buffer b = s % NBUF, with the loads of stage s + NBUF - 1
@@ -1613,86 +1694,101 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
     // as out-of-range loads, so that every stage leaves the same count)
     auto stage = [&]( auto bc, int32_t s ) {
         constexpr int b  = decltype( bc )::value;
-        const float  *SA = smem + b * ( BK * BM ) + 64 * w + 4 * lr;
-        const float  *SB = smem + NBUF * BK * BM + b * ( BK * BN ) + 4 * lr;
-        f4            av[BK / 4], bv[BK / 4];
+        const T      *SA = buffer( bc ) + WR * w + lr;
+        const T      *SB = buffer( bc ) + BK * AST + VB * lr;
+        T             av[BK / 4][RB];
+        bvec          bv[BK / 4][4 / VB];
 #pragma unroll
         for ( int ks = 0; ks < BK / 4; ks++ ) {
-            av[ks] = *(const f4 *)&SA[( 4 * ks + lg ) * BM];
-            bv[ks] = *(const f4 *)&SB[( 4 * ks + lg ) * BN];
+#pragma unroll
+            for ( int i = 0; i < RB; i++ ) av[ks][i] = SA[( 4 * ks + lg ) * AST + 16 * i];
+#pragma unroll
+            for ( int j = 0; j < 4 / VB; j++ ) bv[ks][j] = *(const bvec *)&SB[( 4 * ks + lg ) * BN + 16 * VB * j];
         }
-        if ( NBUF > 2 || s + 1 < ns ) {
-            dma( std::integral_constant<int, ( b + NBUF - 1 ) % NBUF>{}, ( s + NBUF - 1 ) * BK );
+        if constexpr ( LDLT ) {
+#pragma unroll
+            for ( int ks = 0; ks < BK / 4; ks++ ) {
+                const T d = sD[s * BK + 4 * ks + lg];
+#pragma unroll
+                for ( int i = 0; i < RB; i++ ) av[ks][i] = av[ks][i] * d;
+            }
         }
+        dma( std::integral_constant<int, ( b + NBUF - 1 ) % NBUF>{}, ( s + NBUF - 1 ) * BK );
 #pragma unroll
         for ( int ks = 0; ks < BK / 4; ks++ )
 #pragma unroll
-            for ( int i = 0; i < 4; i++ )
+            for ( int i = 0; i < RB; i++ )
 #pragma unroll
-                for ( int j = 0; j < 4; j++ ) acc[i][j] = M::mma( av[ks][i], bv[ks][j], acc[i][j] );
-        // the products stay ahead of the wait for the next stage's loads
-        __builtin_amdgcn_sched_barrier( 0 );
-        __builtin_amdgcn_s_waitcnt( WAIT_NEXT );   // this wave's loads of stage s + 1 are in LDS
-        __syncthreads();
+                for ( int j = 0; j < 4; j++ ) acc[i][j] = M::mma( bv[ks][j / VB].e[j % VB], av[ks][i], acc[i][j] );
+        next_stage();
     };
     dma( std::integral_constant<int, 0>{}, 0 );
-    if constexpr ( NBUF > 2 ) dma( std::integral_constant<int, 1>{}, BK );
-    if constexpr ( NBUF > 3 ) dma( std::integral_constant<int, 2>{}, 2 * BK );
-    __builtin_amdgcn_s_waitcnt( WAIT_NEXT );
-    __syncthreads();
+    dma( std::integral_constant<int, 1>{}, BK );
+    next_stage();
     for ( int32_t s = 0; s < ns; s += NBUF ) {
         stage( std::integral_constant<int, 0>{}, s );
         if ( s + 1 < ns ) stage( std::integral_constant<int, 1>{}, s + 1 );
-        if constexpr ( NBUF > 2 ) {
-            if ( s + 2 < ns ) stage( std::integral_constant<int, 2>{}, s + 2 );
-        }
-        if constexpr ( NBUF > 3 ) {
-            if ( s + 3 < ns ) stage( std::integral_constant<int, 3>{}, s + 3 );
-        }
+        if ( s + 2 < ns ) stage( std::integral_constant<int, 2>{}, s + 2 );
     }
-    if constexpr ( NBUF > 2 ) {
-        // the out-of-range loads past the last stage land before the scatter
-        // reuses the buffers
-        __builtin_amdgcn_s_waitcnt( 0x0F70 );
-        __syncthreads();
-    }
+    // the loads past the last stage land before the workgroup's LDS is given up
+    __builtin_amdgcn_s_waitcnt( 0x0F70 );
 
-    // scatter: slab j holds the columns 4 r + j of the wave's block
-    const bool atomic = ( t.flags & 1 );
-    float     *sE     = smem + w * ( 64 * 17 );
+    // C -= acc, a slab of 16 columns at a time through the wave's own part of
+    // the stage buffers, so that a lane owns a row (LPR lanes to a row) and a
+    // memory instruction covers WR consecutive rows of one column
+    const bool    atomic = ( t.flags & 1 );
+    constexpr int LPR = 64 / WR, CPL = 16 / LPR;             // lanes per row, columns per lane
+    constexpr int CH  = ( CPL < 8 ) ? CPL : 8;               // columns in flight
+    static_assert( WR * 17 <= BK * ( AST + BN ), "a wave's slab fits in a stage buffer" );
+    T *sE = ( w == 0 ) ? stage0 : ( w == 1 ) ? stage1 : stage2;
+    bare_barrier();
+    if constexpr ( 2 * WR * 17 <= BK * ( AST + BN ) ) {
+        sE = ( w == 3 ) ? stage2 + WR * 17 : sE;
+    }
+    else {
+        __shared__ T slab3[WR * 17];
+        sE = ( w == 3 ) ? slab3 : sE;
+    }
+    const int      erow = lane / LPR, epart = lane % LPR;
+    const uint32_t ro = __shfl( dst, ( OWN ? 0 : WR * w ) + ( OWN ? LPE : 1 ) * erow );
+    const uint32_t rl = __shfl( dld, ( OWN ? 0 : WR * w ) + ( OWN ? LPE : 1 ) * erow );
 #pragma unroll
     for ( int j = 0; j < 4; j++ ) {
 #pragma unroll
-        for ( int i = 0; i < 4; i++ )
+        for ( int i = 0; i < RB; i++ )
 #pragma unroll
-            for ( int v = 0; v < 4; v++ ) sE[( 4 * M::row( lane, v ) + i ) * 17 + lr] = M::get( acc[i][j], v );
-        __syncthreads();
-        // two halves of 8 columns (the other slabs' accumulators are live)
+            for ( int v = 0; v < 4; v++ ) sE[( 16 * i + lr ) * 17 + M::row( lane, v )] = M::get( acc[i][j], v );
+        __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
 #pragma unroll
-        for ( int h = 0; h < 16; h += 8 ) {
-            uint32_t off[8];
-            float    val[8];
+        for ( int h = 0; h < CPL; h += CH ) {
+            uint32_t off[CH];
+            T        val[CH];
 #pragma unroll
-            for ( int q = 0; q < 8; q++ ) {
-                const int cc = 4 * ( h + q ) + j;
-                off[q] = ( dst != PXD_OOB && cc < nvalid ) ? dst + (uint32_t)( colF0 + cc ) * dld : PXD_OOB;
-                val[q] = sE[lane * 17 + h + q];
+            for ( int q = 0; q < CH; q++ ) {
+                const int m  = CPL * epart + h + q;
+                const int cc = 16 * VB * ( j / VB ) + VB * m + j % VB;
+                off[q] = ( ro != PXD_OOB && cc < nvalid ) ? ro + (uint32_t)( colF0 + cc ) * rl : PXD_OOB;
+                val[q] = sE[erow * 17 + m];
             }
             if ( atomic ) {
 #pragma unroll
-                for ( int q = 0; q < 8; q++ ) {
+                for ( int q = 0; q < CH; q++ ) {
                     if ( off[q] != PXD_OOB ) px_atomic_add( LC + cf.coefoff + off[q] / ES, -val[q] );
                 }
             }
             else {
-                float old[8];
+                T old[CH];
 #pragma unroll
-                for ( int q = 0; q < 8; q++ ) old[q] = bufio<float>::load( rC, off[q] );
+                for ( int q = 0; q < CH; q++ ) old[q] = bufio<T>::load( rC, off[q] );
 #pragma unroll
-                for ( int q = 0; q < 8; q++ ) bufio<float>::store( old[q] - val[q], rC, off[q] );
+                for ( int q = 0; q < CH; q++ ) bufio<T>::store( old[q] - val[q], rC, off[q] );
             }
         }
-        __syncthreads();
+        __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
     }
     stamp_end( stamps, ti, t_stamp );
 }
