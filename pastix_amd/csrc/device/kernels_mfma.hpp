@@ -1472,12 +1472,20 @@ k_update_big( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
 // of BK k values: while a stage's products run, the loads of the next NBUF - 1
 // stages are in flight, and each stage ends with one barrier.
 //
-// The staged tiles are k major (A[k][BM rows], B[k][64 columns]).  A load
-// instruction moves 64 dwords (one k value of 64 rows of float, of 32 rows of
-// the 8-byte types, whose two dwords go to a lane pair) or 64 elements of 16
-// bytes; every lane writes LDS at its own consecutive place.  Wave w computes
-// the rows [w BM/4, (w+1) BM/4) of the tile and, except in complex double,
-// loads the same ones.
+// Every lane of a load instruction writes LDS at its own consecutive place, 4
+// or 16 bytes; the staged tiles are k major.  Wave w loads and computes the rows
+// [w BM/4, (w+1) BM/4) of A, and the waves share the k values of B.
+//   float: 4 bytes per lane, one k value of the wave's 64 rows (of the 64
+//     columns of B).
+//   8-byte types: where the wave's 32 rows lie in one blok, 16 bytes per lane,
+//     4 k values of all of them (A[wave][k][32 rows]); else 4 bytes per lane,
+//     one k value.  B, whose 64 columns always lie in one blok, 16 bytes per
+//     lane (columns past the update are other values of the cblk, and their
+//     results are dropped).  100^3 double, update launches: 133.6 ms with 4
+//     bytes per lane throughout, 126.1 ms; 80^3 complex64 72.2 -> 70.2 ms.  In
+//     float the same gained nothing (65.4 against 68.0 ms).
+//   complex double: 16 bytes per lane, an element; each wave loads all 64 rows
+//     at its own k value.
 //
 // C -= acc goes a 16-column slab at a time through LDS, each wave for itself,
 // so that a memory instruction covers the wave's 16 to 64 consecutive rows of
@@ -1537,29 +1545,30 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
     constexpr int      BK = dma_shape<T>::bk, NBUF = 3;
     constexpr int      BM = upd_rows<T>::value, BN = PXD_UPD_BN;
     constexpr uint32_t ES = sizeof( T );
-    constexpr int      LPE = ( ES == 8 ) ? 2 : 1;            // lanes per element of a load
-    constexpr int      LSZ = ( ES == 16 ) ? 16 : 4;          // bytes per lane of a load
-    constexpr int      RPI = 64 / LPE;                       // rows (columns of B) per load
+    constexpr int      LPE = ( ES == 8 ) ? 2 : 1;            // lanes per element of a load of one row per lane
     constexpr int      WR  = BM / 4, RB = WR / 16;           // rows and 16-row blocks per wave
-    constexpr bool     OWN = ( RPI == WR );                  // a wave loads its own rows (else all rows of its k)
-    constexpr int      QA  = OWN ? BK : BK / 4;              // loads per stage and wave
-    constexpr int      QB  = BK * BN / RPI / 4;
-    constexpr int      BG  = BN / RPI;                       // loads per k value of B
-    constexpr int      AST = BM + ( ES == 4 ? 16 : 0 );      // float: k values 64 bytes apart, else two meet in a bank
-    constexpr int      LPS = QA + QB;
-    constexpr int      VMN = LPS * ( NBUF - 2 );             // loads issued after the next stage's
-    static_assert( BK % 4 == 0, "stages of whole 4-k products" );
-    static_assert( OWN || RPI == BM, "a load covers a wave's rows or the whole tile's" );
-    static_assert( VMN < 64, "vmcnt holds 6 bits" );
-    static_assert( sizeof( search_keys ) <= BK * AST * ES, "search keys fit in one A buffer" );
-    constexpr int WAIT_NEXT = ( VMN & 15 ) | ( ( VMN >> 4 ) << 14 ) | 0x0F70;   // s_waitcnt vmcnt(VMN)
+    constexpr bool     OWN = ( ES < 16 );                    // a wave loads its own rows (else all rows of its k)
+    constexpr bool     W16 = ( ES == 8 );                    // 16 bytes per lane where the rows allow it
+    constexpr int      QW  = BK / 4;                         // ... loads of A per stage and wave
+    constexpr int      QN  = OWN ? BK : BK / 4;              // and one row per lane (pair)
+    constexpr int      AST = W16 ? WR : BM + ( ES == 4 ? 16 : 0 );   // elements between the k values of A
+                                                             // (float: 64 bytes more, else two meet in a bank)
+    constexpr int      SA0 = W16 ? BK * WR : WR;             // ... and between the waves' rows
+    constexpr int      ASZ = W16 ? BK * BM : BK * AST;       // elements of A in a stage
+    constexpr int      BL  = ( ES == 4 ) ? 4 : 16;           // bytes per lane of a load of B
+    constexpr int      BE  = BL / (int)ES, KB = 64 * BE / BN;   // elements per lane, k values per load
+    constexpr int      QB  = BK / KB / 4;                    // loads of B per stage and wave
+    static_assert( BK % 4 == 0 && QB * KB * 4 == BK, "stages of whole 4-k products" );
+    static_assert( !W16 || WR * ES == 256, "16 lanes hold a wave's rows in 16 bytes each" );
+    static_assert( sizeof( search_keys ) <= ASZ * ES, "search keys fit in one A buffer" );
     constexpr int DN = PXD_TRSM_NT * 16 + BK;
+    constexpr int SE = ASZ + BK * BN;   // elements of a stage
     // one variable per stage (A, then B): the compiler tells loads into one
     // from reads of another only by the variable, and waits for all of them
     // where it cannot
-    __shared__ __align__( 16 ) T stage0[BK * ( AST + BN )];
-    __shared__ __align__( 16 ) T stage1[BK * ( AST + BN )];
-    __shared__ __align__( 16 ) T stage2[BK * ( AST + BN )];
+    __shared__ __align__( 16 ) T stage0[SE];
+    __shared__ __align__( 16 ) T stage1[SE];
+    __shared__ __align__( 16 ) T stage2[SE];
     T *sD = nullptr;
     if constexpr ( LDLT ) {
         __shared__ T sDk[DN];
@@ -1611,16 +1620,20 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
     }
     __syncthreads();
 
-    // the lane's row of the tile: byte offset of its part of the first element
-    // and byte stride between its columns in the source, and its place in F
-    uint32_t abase = PXD_OOB, astep = 0, dst = PXD_OOB, dld = 0;
+    // the lane's row of the tile (complex double: every wave all rows, its own
+    // the same place): its blok's stacked offset, its place in the blok and
+    // the byte stride between its columns in the source, its place in F
+    const int r0w   = t.tm * BM + ( OWN ? WR * w : 0 );
+    int32_t   boff = 0, ain = 0;
+    uint32_t  astep = 0, dst = PXD_OOB, dld = 0;
     {
-        const int32_t r = t.tm * BM + ( OWN ? WR * w : 0 ) + lane / LPE;
+        const int32_t r = r0w + lane / LPE;
         if ( r < Mr ) {
             const int32_t s  = r0 + r;
             const dblok   ib = bk[search_row( sk, bk, t.blok, lb, s )];
             const int32_t g  = ib.frownum + ( s - ib.rowoff );
-            abase = (uint32_t)( ib.rowoff * K + ( s - ib.rowoff ) ) * ES + LSZ * ( lane % LPE );
+            boff  = ib.rowoff;
+            ain   = s - ib.rowoff;
             astep = (uint32_t)( ib.lrownum - ib.frownum + 1 ) * ES;
             const dblok fb = bk[search_grow( sk, bk, cf.fblok, flb, g )];
             if ( g >= fb.frownum && g <= fb.lrownum ) {
@@ -1629,37 +1642,54 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
             }
         }
     }
-    // the lane's facing column: wave w loads the columns of group w % BG at
-    // the k values w / BG, w / BG + 4 / BG, ... of a stage
-    constexpr int  KSB    = 4 / BG;
-    const int32_t  nvalid = min( BN, N - t.tn * BN );
-    const int      bcol   = RPI * ( w % BG ) + lane / LPE, bk0 = w / BG;
-    uint32_t       bo = PXD_OOB, bstep = 0;
-    if ( bcol < nvalid ) {
-        bo    = (uint32_t)( bb.rowoff * K + t.tn * BN + bcol ) * ES + LSZ * ( lane % LPE ) + (uint32_t)( bk0 * N ) * ES;
-        bstep = (uint32_t)( KSB * N ) * ES;
+    // the wave's rows in one blok: the row of lane 0 and the last one inside
+    // the update (rows past it read what follows, and are dropped)
+    const int  lastl = LPE * min( WR - 1, Mr - 1 - r0w );
+    const bool wide  = W16 && lastl >= 0 &&
+                      __builtin_amdgcn_readfirstlane( boff ) == __builtin_amdgcn_readlane( boff, max( 0, lastl ) );
+    uint32_t ao = PXD_OOB;
+    int      ak0 = OWN ? 0 : w;   // the lane's first k value of a stage
+    if ( wide ) {
+        ak0   = lane >> 4;
+        astep = __builtin_amdgcn_readfirstlane( astep );
+        ao    = (uint32_t)( __builtin_amdgcn_readfirstlane( boff ) * K + __builtin_amdgcn_readfirstlane( ain ) ) * ES +
+             16 * ( lane & 15 ) + ak0 * astep;
+        astep *= 4;
     }
-    const int ak0 = OWN ? 0 : w;
-    uint32_t  ao = ( abase == PXD_OOB ) ? PXD_OOB : abase + (uint32_t)ak0 * astep;
-    if constexpr ( !OWN ) astep *= 4;
+    else if ( r0w + lane / LPE < Mr ) {
+        ao = (uint32_t)( boff * K + ain ) * ES + 4 * ( lane % LPE ) + ak0 * astep;
+        if constexpr ( !OWN ) astep *= 4;
+    }
+    // the lane's columns of B, at the k values KB (w + 4 q) + lane / (lanes per k)
+    const int32_t  nvalid = min( BN, N - t.tn * BN );
+    const int      bcol   = BE * ( lane % ( BN / BE ) ), bk0 = KB * w + lane / ( BN / BE );
+    const uint32_t bstep  = (uint32_t)( 4 * KB * N ) * ES;
+    uint32_t       bo     = (uint32_t)( bb.rowoff * K + t.tn * BN + bcol + bk0 * N ) * ES;
 
     // stage k0 into buffer b; the offsets advance from load to load, so that
     // no per-k products stay live across the loop
     auto dma = [&]( auto bc, int32_t k0 ) {
-        T            *dA = buffer( bc ) + ( OWN ? WR * w : w * AST );
-        T            *dB = buffer( bc ) + BK * AST + bk0 * BN + RPI * ( w % BG );
-        const bool    full = ( k0 + BK <= K );
+        T         *dA   = buffer( bc ) + ( OWN ? SA0 * w : AST * w );
+        T         *dB   = buffer( bc ) + ASZ + KB * BN * w;
+        const bool full = ( k0 + BK <= K );
+        if ( W16 && wide ) {
 #pragma unroll
-        for ( int q = 0; q < QA; q++ ) {
-            constexpr int  KSA = OWN ? 1 : 4;
-            const uint32_t o = ( full || k0 + KSA * q + ak0 < K ) ? ao : PXD_OOB;
-            load_lds<LSZ>( rA, dA + KSA * q * AST, o );
-            ao += astep;
+            for ( int q = 0; q < QW; q++ ) {
+                load_lds<16>( rA, dA + 4 * q * AST, ( full || k0 + 4 * q + ak0 < K ) ? ao : PXD_OOB );
+                ao += astep;
+            }
+        }
+        else {
+#pragma unroll
+            for ( int q = 0; q < QN; q++ ) {
+                constexpr int KS = OWN ? 1 : 4;
+                load_lds<OWN ? 4 : 16>( rA, dA + KS * q * AST, ( full || k0 + KS * q + ak0 < K ) ? ao : PXD_OOB );
+                ao += astep;
+            }
         }
 #pragma unroll
         for ( int q = 0; q < QB; q++ ) {
-            const uint32_t o = ( full || k0 + KSB * q + bk0 < K ) ? bo : PXD_OOB;
-            load_lds<LSZ>( rB, dB + KSB * q * BN, o );
+            load_lds<BL>( rB, dB + 4 * KB * BN * q, ( full || k0 + 4 * KB * q + bk0 < K ) ? bo : PXD_OOB );
             bo += bstep;
         }
     };
@@ -1676,17 +1706,26 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
     // the stage has returned.  Not __syncthreads(): its fence waits for the
     // loads in flight too (vmcnt 0), which leaves no stage ahead of the
     // products.
-    auto next_stage = []() {
+    auto next_stage = [&]() {
         __builtin_amdgcn_sched_barrier( 0 );
-        __builtin_amdgcn_s_waitcnt( WAIT_NEXT );
+        static_assert( QN + QB < 16, "4 bits of vmcnt" );
+        if ( W16 && wide ) {
+            __builtin_amdgcn_s_waitcnt( 0x0F70 | ( QW + QB ) );   // vmcnt: the loads of one stage
+        }
+        else {
+            __builtin_amdgcn_s_waitcnt( 0x0F70 | ( QN + QB ) );
+        }
         bare_barrier();
         __builtin_amdgcn_sched_barrier( 0 );
     };
 
     // 16-byte reads of B: VB columns next to each other feed VB of the four
-    // column tiles (tile j holds the columns 16 VB (j / VB) + VB r + j % VB)
+    // column tiles (tile j holds the columns 16 VB (j / VB) + VB r + j % VB),
+    // and of A in the 8-byte types: block i holds the rows 2 r + i of the
+    // wave's (elsewhere 16 i + r)
     constexpr int VB = 16 / ES;
     struct __align__( 16 ) bvec { T e[VB]; };
+    static_assert( RB == VB, "a lane's rows fill 16 bytes" );
     const int     lr = lane & 15, lg = lane >> 4;
     const int32_t ns = ( K + BK - 1 ) / BK;
     // stage s from buffer b = s % NBUF, with the loads of stage s + NBUF - 1
@@ -1694,14 +1733,18 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
     // as out-of-range loads, so that every stage leaves the same count)
     auto stage = [&]( auto bc, int32_t s ) {
         constexpr int b  = decltype( bc )::value;
-        const T      *SA = buffer( bc ) + WR * w + lr;
-        const T      *SB = buffer( bc ) + BK * AST + VB * lr;
-        T             av[BK / 4][RB];
-        bvec          bv[BK / 4][4 / VB];
+        const T      *SA = buffer( bc ) + SA0 * w + ( W16 ? VB : 1 ) * lr;
+        const T      *SB = buffer( bc ) + ASZ + VB * lr;
+        bvec          av[BK / 4], bv[BK / 4][4 / VB];
 #pragma unroll
         for ( int ks = 0; ks < BK / 4; ks++ ) {
+            if constexpr ( W16 ) {
+                av[ks] = *(const bvec *)&SA[( 4 * ks + lg ) * AST];
+            }
+            else {
 #pragma unroll
-            for ( int i = 0; i < RB; i++ ) av[ks][i] = SA[( 4 * ks + lg ) * AST + 16 * i];
+                for ( int i = 0; i < RB; i++ ) av[ks].e[i] = SA[( 4 * ks + lg ) * AST + 16 * i];
+            }
 #pragma unroll
             for ( int j = 0; j < 4 / VB; j++ ) bv[ks][j] = *(const bvec *)&SB[( 4 * ks + lg ) * BN + 16 * VB * j];
         }
@@ -1710,7 +1753,7 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
             for ( int ks = 0; ks < BK / 4; ks++ ) {
                 const T d = sD[s * BK + 4 * ks + lg];
 #pragma unroll
-                for ( int i = 0; i < RB; i++ ) av[ks][i] = av[ks][i] * d;
+                for ( int i = 0; i < RB; i++ ) av[ks].e[i] = av[ks].e[i] * d;
             }
         }
         dma( std::integral_constant<int, ( b + NBUF - 1 ) % NBUF>{}, ( s + NBUF - 1 ) * BK );
@@ -1719,7 +1762,7 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
 #pragma unroll
             for ( int i = 0; i < RB; i++ )
 #pragma unroll
-                for ( int j = 0; j < 4; j++ ) acc[i][j] = M::mma( bv[ks][j / VB].e[j % VB], av[ks][i], acc[i][j] );
+                for ( int j = 0; j < 4; j++ ) acc[i][j] = M::mma( bv[ks][j / VB].e[j % VB], av[ks].e[i], acc[i][j] );
         next_stage();
     };
     dma( std::integral_constant<int, 0>{}, 0 );
@@ -1739,10 +1782,10 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
     const bool    atomic = ( t.flags & 1 );
     constexpr int LPR = 64 / WR, CPL = 16 / LPR;             // lanes per row, columns per lane
     constexpr int CH  = ( CPL < 8 ) ? CPL : 8;               // columns in flight
-    static_assert( WR * 17 <= BK * ( AST + BN ), "a wave's slab fits in a stage buffer" );
+    static_assert( WR * 17 <= SE, "a wave's slab fits in a stage buffer" );
     T *sE = ( w == 0 ) ? stage0 : ( w == 1 ) ? stage1 : stage2;
     bare_barrier();
-    if constexpr ( 2 * WR * 17 <= BK * ( AST + BN ) ) {
+    if constexpr ( 2 * WR * 17 <= SE ) {
         sE = ( w == 3 ) ? stage2 + WR * 17 : sE;
     }
     else {
@@ -1757,7 +1800,7 @@ k_update_dma( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
 #pragma unroll
         for ( int i = 0; i < RB; i++ )
 #pragma unroll
-            for ( int v = 0; v < 4; v++ ) sE[( 16 * i + lr ) * 17 + M::row( lane, v )] = M::get( acc[i][j], v );
+            for ( int v = 0; v < 4; v++ ) sE[( W16 ? VB * lr + i : 16 * i + lr ) * 17 + M::row( lane, v )] = M::get( acc[i][j], v );
         __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
