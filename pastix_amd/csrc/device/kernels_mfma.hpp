@@ -9,8 +9,8 @@
 #pragma once
 #include "kernels_fact.hpp"
 #include "kernels_solve.hpp"
-#include "mfma.hpp"
 #include <type_traits>
+#include "kernels_elim.hpp"
 
 // tasks of the block-column inversion: cblk and first column of the block
 struct inv_task {
@@ -38,314 +38,6 @@ tri_index( int idx, int &i, int &j )
     if ( ( i + 1 ) * ( i + 2 ) / 2 <= idx ) i++;
     if ( i * ( i + 1 ) / 2 > idx ) i--;
     j = idx - i * ( i + 1 ) / 2;
-}
-
-// Unblocked eliminations of a 32 x 32 diagonal block in LDS (s[col][row],
-// zero beyond bs rows and columns), one barrier per elimination step.  Each
-// of the 256 threads keeps four entries of the block and of each inverse in
-// registers: row r = tid & 31, columns g, g + 8, g + 16, g + 24 (g = tid >>
-// 5).  The column and rows that a step reads go through a double-buffered
-// exchange area x in LDS (4 rows of 32 for the symmetric forms, 8 for LU),
-// written by their owners before the step's barrier.  On return the block and the inverses are back in LDS,
-// sD holds the pivots, and the result is the number of replaced pivots
-// (counted by thread 0 only; the other threads return 0).
-static_assert( PXD_THREADS == 8 * PXD_NB, "the elimination maps 256 threads on a 32 x 32 block" );
-
-template <typename T>
-__device__ inline T
-pick4( T v0, T v1, T v2, T v3, int u )
-{
-    return ( u == 0 ) ? v0 : ( u == 1 ) ? v1 : ( u == 2 ) ? v2 : v3;
-}
-
-// Complex double: each LDS read of a step as it is needed (the read-ahead
-// form below would not fit the register file of the panel kernels).
-template <typename T, bool LDLT>
-__device__ inline int
-elim_sym32_single( T ( *sA )[PXD_NB + 1], T ( *sI )[PXD_NB + 1], T *sD, T ( *x )[PXD_NB], int bs,
-            typename px_real<T>::type tau, int tid )
-{
-    typedef typename px_real<T>::type R;
-    const int r = tid & ( PXD_NB - 1 ), g = tid >> 5;
-    T a[4], w[4];
-#pragma unroll
-    for ( int u = 0; u < 4; u++ ) {
-        a[u] = sA[g + 8 * u][r];
-        w[u] = sI[g + 8 * u][r];
-    }
-    int piv = 0;
-    for ( int cc = 0; cc < bs; cc++ ) {
-        T *colA = x[2 * ( cc & 1 )], *rowW = x[2 * ( cc & 1 ) + 1];
-        if ( g == ( cc & 7 ) ) {
-            colA[r] = pick4( a[0], a[1], a[2], a[3], cc >> 3 );   // column cc of A
-        }
-        if ( r == cc ) {
-#pragma unroll
-            for ( int u = 0; u < 4; u++ ) {
-                rowW[g + 8 * u] = w[u];      // row cc of W
-            }
-        }
-        __syncthreads();
-        T d = colA[cc];
-        if ( px_abs( d ) < tau ) {
-            d = ( LDLT && px_re( d ) < (R)0 ) ? (T)-tau : (T)tau;
-            piv += ( tid == 0 );
-        }
-        const T rinv = (T)1 / d;
-        if ( r > cc && r < bs ) {
-            const T ar = colA[r];
-#pragma unroll
-            for ( int u = 0; u < 4; u++ ) {
-                const int c = g + 8 * u;
-                if ( c > cc && c <= r ) {
-                    a[u] -= ar * colA[c] * rinv;
-                }
-                else if ( c <= cc ) {
-                    w[u] -= ar * rinv * rowW[c];
-                }
-            }
-        }
-        if ( tid == 0 ) {
-            sD[cc] = d;
-        }
-    }
-#pragma unroll
-    for ( int u = 0; u < 4; u++ ) {
-        sA[g + 8 * u][r] = a[u];
-        sI[g + 8 * u][r] = w[u];
-    }
-    __syncthreads();
-    return piv;
-}
-
-// Symmetric: A = U D U^T, U unit lower with multipliers u_rc = a_rc / d_c,
-// on the lower triangle of sA; the same row operations on W = I (sI) leave
-// W = U^{-1}.  A pivot below tau in modulus becomes tau (Cholesky,
-// core_zpotf2sp) or sign(re d) tau (LDL^T, core_zsytf2sp).
-template <typename T, bool LDLT>
-__device__ inline int
-elim_sym32_ahead( T ( *sA )[PXD_NB + 1], T ( *sI )[PXD_NB + 1], T *sD, T ( *x )[PXD_NB], int bs,
-            typename px_real<T>::type tau, int tid )
-{
-    typedef typename px_real<T>::type R;
-    const int r = tid & ( PXD_NB - 1 ), g = tid >> 5;
-    T a[4], w[4];
-#pragma unroll
-    for ( int u = 0; u < 4; u++ ) {
-        a[u] = sA[g + 8 * u][r];
-        w[u] = sI[g + 8 * u][r];
-    }
-    int piv = 0;
-    for ( int cc = 0; cc < bs; cc++ ) {
-        T *colA = x[2 * ( cc & 1 )], *rowW = x[2 * ( cc & 1 ) + 1];
-        if ( g == ( cc & 7 ) ) {
-            colA[r] = pick4( a[0], a[1], a[2], a[3], cc >> 3 );   // column cc of A
-        }
-        if ( r == cc ) {
-#pragma unroll
-            for ( int u = 0; u < 4; u++ ) {
-                rowW[g + 8 * u] = w[u];      // row cc of W
-            }
-        }
-        __syncthreads();
-        // every read of the step at once, then the updates as selects: one
-        // LDS round trip per step
-        T d = colA[cc];
-        const T ar = colA[r];
-        T ca[4], rw[4];
-#pragma unroll
-        for ( int u = 0; u < 4; u++ ) {
-            ca[u] = colA[g + 8 * u];
-            rw[u] = rowW[g + 8 * u];
-        }
-        if ( px_abs( d ) < tau ) {
-            d = ( LDLT && px_re( d ) < (R)0 ) ? (T)-tau : (T)tau;
-            piv += ( tid == 0 );
-        }
-        const T    rinv = (T)1 / d;
-        const bool act  = r > cc && r < bs;
-#pragma unroll
-        for ( int u = 0; u < 4; u++ ) {
-            const int c  = g + 8 * u;
-            const T   na = a[u] - ar * ca[u] * rinv;
-            const T   nw = w[u] - ar * rinv * rw[u];
-            a[u] = ( act && c > cc && c <= r ) ? na : a[u];
-            w[u] = ( act && c <= cc ) ? nw : w[u];
-        }
-        if ( tid == 0 ) {
-            sD[cc] = d;
-        }
-    }
-#pragma unroll
-    for ( int u = 0; u < 4; u++ ) {
-        sA[g + 8 * u][r] = a[u];
-        sI[g + 8 * u][r] = w[u];
-    }
-    __syncthreads();
-    return piv;
-}
-
-template <typename T, bool LDLT>
-__device__ inline int
-elim_sym32( T ( *sA )[PXD_NB + 1], T ( *sI )[PXD_NB + 1], T *sD, T ( *x )[PXD_NB], int bs,
-            typename px_real<T>::type tau, int tid )
-{
-    if constexpr ( sizeof( T ) > 8 ) {
-        return elim_sym32_single<T, LDLT>( sA, sI, sD, x, bs, tau, tid );
-    }
-    else {
-        return elim_sym32_ahead<T, LDLT>( sA, sI, sD, x, bs, tau, tid );
-    }
-}
-
-// LU without pivoting: multipliers a_r,cc / d left unscaled in sA; the row
-// operations of L on W_L = I (sIL) leave L11^{-1}, those of U11^T = U~ D on
-// W_U = I (sIU) leave U~^{-1}.  A pivot below tau becomes sign(re d) tau.
-template <typename T>
-__device__ inline int
-elim_lu32_ahead( T ( *sA )[PXD_NB + 1], T ( *sIL )[PXD_NB + 1], T ( *sIU )[PXD_NB + 1], T *sD, T ( *x )[PXD_NB],
-           int bs, typename px_real<T>::type tau, int tid )
-{
-    typedef typename px_real<T>::type R;
-    const int r = tid & ( PXD_NB - 1 ), g = tid >> 5;
-    T a[4], wl[4], wu[4];
-#pragma unroll
-    for ( int u = 0; u < 4; u++ ) {
-        a[u]  = sA[g + 8 * u][r];
-        wl[u] = sIL[g + 8 * u][r];
-        wu[u] = sIU[g + 8 * u][r];
-    }
-    int piv = 0;
-    for ( int cc = 0; cc < bs; cc++ ) {
-        T *colA = x[4 * ( cc & 1 )], *rowA = x[4 * ( cc & 1 ) + 1];
-        T *rowL = x[4 * ( cc & 1 ) + 2], *rowU = x[4 * ( cc & 1 ) + 3];
-        if ( g == ( cc & 7 ) ) {
-            colA[r] = pick4( a[0], a[1], a[2], a[3], cc >> 3 );
-        }
-        if ( r == cc ) {
-#pragma unroll
-            for ( int u = 0; u < 4; u++ ) {
-                rowA[g + 8 * u] = a[u];
-                rowL[g + 8 * u] = wl[u];
-                rowU[g + 8 * u] = wu[u];
-            }
-        }
-        __syncthreads();
-        T d = colA[cc];
-        const T cr = colA[r], rr = rowA[r];
-        T ra[4], rl[4], ru[4];
-#pragma unroll
-        for ( int u = 0; u < 4; u++ ) {
-            ra[u] = rowA[g + 8 * u];
-            rl[u] = rowL[g + 8 * u];
-            ru[u] = rowU[g + 8 * u];
-        }
-        if ( px_abs( d ) < tau ) {
-            d = ( px_re( d ) < (R)0 ) ? (T)-tau : (T)tau;
-            piv += ( tid == 0 );
-        }
-        const T    rinv = (T)1 / d;
-        const bool act  = r > cc && r < bs;
-#pragma unroll
-        for ( int u = 0; u < 4; u++ ) {
-            const int c  = g + 8 * u;
-            const T   na = a[u] - cr * rinv * ra[u];
-            const T   nl = wl[u] - cr * rinv * rl[u];
-            const T   nu = wu[u] - rr * rinv * ru[u];
-            a[u]  = ( act && c > cc && c < bs ) ? na : a[u];
-            wl[u] = ( act && c <= cc ) ? nl : wl[u];
-            wu[u] = ( act && c <= cc ) ? nu : wu[u];
-        }
-        if ( tid == 0 ) {
-            sD[cc] = d;
-        }
-    }
-#pragma unroll
-    for ( int u = 0; u < 4; u++ ) {
-        sA[g + 8 * u][r]  = a[u];
-        sIL[g + 8 * u][r] = wl[u];
-        sIU[g + 8 * u][r] = wu[u];
-    }
-    __syncthreads();
-    return piv;
-}
-
-// complex double: each LDS read as it is needed (register file)
-template <typename T>
-__device__ inline int
-elim_lu32_lean( T ( *sA )[PXD_NB + 1], T ( *sIL )[PXD_NB + 1], T ( *sIU )[PXD_NB + 1], T *sD, T ( *x )[PXD_NB],
-           int bs, typename px_real<T>::type tau, int tid )
-{
-    typedef typename px_real<T>::type R;
-    const int r = tid & ( PXD_NB - 1 ), g = tid >> 5;
-    T a[4], wl[4], wu[4];
-#pragma unroll
-    for ( int u = 0; u < 4; u++ ) {
-        a[u]  = sA[g + 8 * u][r];
-        wl[u] = sIL[g + 8 * u][r];
-        wu[u] = sIU[g + 8 * u][r];
-    }
-    int piv = 0;
-    for ( int cc = 0; cc < bs; cc++ ) {
-        T *colA = x[4 * ( cc & 1 )], *rowA = x[4 * ( cc & 1 ) + 1];
-        T *rowL = x[4 * ( cc & 1 ) + 2], *rowU = x[4 * ( cc & 1 ) + 3];
-        if ( g == ( cc & 7 ) ) {
-            colA[r] = pick4( a[0], a[1], a[2], a[3], cc >> 3 );
-        }
-        if ( r == cc ) {
-#pragma unroll
-            for ( int u = 0; u < 4; u++ ) {
-                rowA[g + 8 * u] = a[u];
-                rowL[g + 8 * u] = wl[u];
-                rowU[g + 8 * u] = wu[u];
-            }
-        }
-        __syncthreads();
-        T d = colA[cc];
-        if ( px_abs( d ) < tau ) {
-            d = ( px_re( d ) < (R)0 ) ? (T)-tau : (T)tau;
-            piv += ( tid == 0 );
-        }
-        const T rinv = (T)1 / d;
-        if ( r > cc && r < bs ) {
-            const T cr = colA[r], rr = rowA[r];
-#pragma unroll
-            for ( int u = 0; u < 4; u++ ) {
-                const int c = g + 8 * u;
-                if ( c > cc && c < bs ) {
-                    a[u] -= cr * rinv * rowA[c];
-                }
-                else if ( c <= cc ) {
-                    wl[u] -= cr * rinv * rowL[c];
-                    wu[u] -= rr * rinv * rowU[c];
-                }
-            }
-        }
-        if ( tid == 0 ) {
-            sD[cc] = d;
-        }
-    }
-#pragma unroll
-    for ( int u = 0; u < 4; u++ ) {
-        sA[g + 8 * u][r]  = a[u];
-        sIL[g + 8 * u][r] = wl[u];
-        sIU[g + 8 * u][r] = wu[u];
-    }
-    __syncthreads();
-    return piv;
-}
-
-template <typename T>
-__device__ inline int
-elim_lu32( T ( *sA )[PXD_NB + 1], T ( *sIL )[PXD_NB + 1], T ( *sIU )[PXD_NB + 1], T *sD, T ( *x )[PXD_NB],
-           int bs, typename px_real<T>::type tau, int tid )
-{
-    if constexpr ( sizeof( T ) > 8 ) {
-        return elim_lu32_lean<T>( sA, sIL, sIU, sD, x, bs, tau, tid );
-    }
-    else {
-        return elim_lu32_ahead<T>( sA, sIL, sIU, sD, x, bs, tau, tid );
-    }
 }
 
 // Per-workgroup timing for the kernel timing log: when stamps is not null,
@@ -420,7 +112,6 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
     __shared__ T sA[PXD_NB][PXD_NB + 1];   // sA[col][row]
     __shared__ T sI[PXD_NB][PXD_NB + 1];   // inverse, sI[col][row]
     __shared__ T sD[PXD_NB];
-    __shared__ T sX[4][PXD_NB];             // exchange area of the elimination
     // L21 of the current block, sP[row][k]: dynamic LDS for the widest cblk of the launch
     extern __shared__ unsigned char smem_raw[];
     T ( *sP )[PXD_NB + 1] = reinterpret_cast<T ( * )[PXD_NB + 1]>( smem_raw );
@@ -458,7 +149,10 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
         __syncthreads();
 
         // unblocked elimination A = U D U^T, W = U^{-1} alongside
-        piv += elim_sym32<T, false>( sA, sI, sD, sX, bs, tau, tid );
+        if ( tid < 64 ) {
+            piv += elim32<T, false, false>( sA, sI, nullptr, sD, bs, tau, tid );
+        }
+        __syncthreads();
         // Cholesky: L = U D^{1/2}, the columns scaled by 1/sqrt(pivot), and
         // L^{-1} = D^{-1/2} U^{-1}, the rows of W scaled likewise.
         for ( int idx = tid; idx < PXD_NB * PXD_NB; idx += PXD_THREADS ) {

@@ -229,7 +229,6 @@ k_panel( const pan_task *__restrict__ tasks, const dcblk *__restrict__ cb, T *L,
         sZ = sZ_lu;
     }
     __shared__ T      sD[NB];
-    __shared__ T      sE[LU ? 8 : 4][NB];   // exchange area of the elimination
 
     const pan_task tk      = tasks[blockIdx.x];
     const uint64_t t_stamp = stamp_begin( stamps );
@@ -415,13 +414,11 @@ k_panel( const pan_task *__restrict__ tasks, const dcblk *__restrict__ cb, T *L,
     }
     __syncthreads();
     const R tau = (R)thresh;
-    int     piv;
-    if constexpr ( LU ) {
-        piv = elim_lu32<T>( sA, sI, sZ, sD, sE, bs, tau, tid );
+    int     piv = 0;
+    if ( w == 0 ) {
+        piv = elim32<T, KIND != PAN_LLT, LU>( sA, sI, sZ, sD, bs, tau, lane );
     }
-    else {
-        piv = elim_sym32<T, KIND == PAN_LDLT>( sA, sI, sD, sE, bs, tau, tid );
-    }
+    __syncthreads();
     // Cholesky: L = U D^{1/2}, L^{-1} = D^{-1/2} U^{-1}.  LDL^T: L = U, the
     // diagonal holds D, the upper part D L^T (the unscaled columns).  LU: the
     // multipliers are scaled by the pivots, and (U^T)^{-1} = D^{-1} W_U; the

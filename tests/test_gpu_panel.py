@@ -1,7 +1,7 @@
 """The diagonal tiles (factorization and inverse, several workgroups per
-tile) at the widths where their 32-column blocks end: one block, one column
-more, two and three blocks and one column more, for every factorization and
-arithmetic.  A two-dimensional grid of (w + 3) x w nodes has a top separator
+tile) at the widths where their 32-column blocks and the 16-column halves of
+an elimination end: half a block, one block, one column more, two and three
+blocks and one column more, for every factorization and arithmetic.  A two-dimensional grid of (w + 3) x w nodes has a top separator
 of exactly w columns."""
 import numpy as np
 import pytest
@@ -19,7 +19,7 @@ KINDS = [("lap7", px.PastixFactPOTRF, np.float64), ("lap7", px.PastixFactPOTRF, 
          ("helmholtz7", px.PastixFactLU, np.complex128), ("helmholtz7", px.PastixFactLU, np.complex64)]
 
 
-@pytest.mark.parametrize("width", [31, 32, 33, 65, 97])
+@pytest.mark.parametrize("width", [15, 16, 17, 31, 32, 33, 65, 97])
 @pytest.mark.parametrize("kind,facto,dtype", KINDS)
 def test_tiles_and_solve_at_block_edges(kind, facto, dtype, width):
     spm = make_problem(kind, width + 3, width, 1)
