@@ -959,17 +959,12 @@ factorize( pxd_ctx_t *ctx, double thresh, int64_t *nbpivots )
         if ( !nt ) {
             return;
         }
-        if ( lu ) {
-            // L_off <- L_off U_kk^{-1};  U^T_off <- U^T_off L_kk^{-T}
-            hipLaunchKernelGGL( ( k_trsm_mfma<T> ), dim3( nt ), dim3( PXD_THREADS ), 0, st, ctx->dtrsm + lv.t0,
-                                ctx->dcb, ctx->dbk, L, (const T *)DU, 0, stp( st_trsm, lv.t0, 0, n_trsm ), ctx->prio );
-            hipLaunchKernelGGL( ( k_trsm_mfma<T> ), dim3( nt ), dim3( PXD_THREADS ), 0, st, ctx->dtrsm + lv.t0,
-                                ctx->dcb, ctx->dbk, U, (const T *)DI, 0, stp( st_trsm, lv.t0, 1, n_trsm ), ctx->prio );
-            launches++;
-        }
-        else if ( ctx->kernels ) {
-            hipLaunchKernelGGL( ( k_trsm_mfma<T> ), dim3( nt ), dim3( PXD_THREADS ), 0, st, ctx->dtrsm + lv.t0,
-                                ctx->dcb, ctx->dbk, L, (const T *)DI, ldlt, stp( st_trsm, lv.t0, 0, n_trsm ), ctx->prio );
+        if ( ctx->kernels ) {
+            // LU: L_off <- L_off U_kk^{-1} and U^T_off <- U^T_off L_kk^{-T}
+            hipLaunchKernelGGL( ( k_trsm_mfma<T> ), dim3( lu ? 2 * nt : nt ), dim3( PXD_THREADS ), 0, st,
+                                ctx->dtrsm + lv.t0, (int32_t)nt, ctx->dcb, ctx->dbk, L, (const T *)DU, U,
+                                (const T *)DI, ldlt, stp( st_trsm, lv.t0, 0, n_trsm ), stp( st_trsm, lv.t0, 1, n_trsm ),
+                                ctx->prio );
         }
         else if constexpr ( std::is_same<T, typename px_real<T>::type>::value ) {
             if ( ctx->trsm_rt == 32 ) {

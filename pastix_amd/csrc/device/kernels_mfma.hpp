@@ -461,6 +461,10 @@ k_trtri( const inv_task *__restrict__ tasks, const dcblk *__restrict__ cb, const
 // of an MFMA step are permuted (lane group g takes k = KV*g + s) so that
 // every fragment is one 16-byte read.  Stages whose k range lies above a
 // column tile (Linv zero there) are skipped for that tile.
+// LU takes its two sides (L with the inverses of the U_kk^T, U^T with those of
+// the L_kk) in one launch: one after the other, each left most of the chip idle
+// at the top of the tree. TRSM launches alone, 64^3 float 4.87 ->
+// 3.49 ms, 41^3 double 1.93 -> 1.14 ms.
 template <typename T> struct trsm_cpw;
 template <> struct trsm_cpw<float>  { static constexpr int value = 2; };
 template <> struct trsm_cpw<double> { static constexpr int value = 2; };
@@ -469,9 +473,10 @@ template <> struct trsm_cpw<pxcd>   { static constexpr int value = 1; };
 
 template <typename T>
 __global__ void __launch_bounds__( PXD_THREADS, 2 )
-k_trsm_mfma( const row_task *__restrict__ tasks, const dcblk *__restrict__ cb,
-             const dblok *__restrict__ bk, T *__restrict__ L, const T *__restrict__ Linv, int ldlt,
-             uint64_t *__restrict__ stamps, int prio )
+k_trsm_mfma( const row_task *__restrict__ tasks, int32_t ntasks, const dcblk *__restrict__ cb,
+             const dblok *__restrict__ bk, T *__restrict__ L0, const T *__restrict__ Linv0, T *__restrict__ L1,
+             const T *__restrict__ Linv1, int ldlt, uint64_t *__restrict__ stamps0, uint64_t *__restrict__ stamps1,
+             int prio )
 {
     typedef mfma16<T>                 M;
     typedef typename M::acc_t         acc_t;
@@ -490,8 +495,14 @@ k_trsm_mfma( const row_task *__restrict__ tasks, const dcblk *__restrict__ cb,
     __shared__ int32_t sLd[64];
     __shared__ T       sDi[PXD_TRSM_NT * 16];        // LDL^T: 1 / D of the cblk
 
-    const int32_t  ti   = xcd_task( blockIdx.x, gridDim.x );
-    const row_task t    = tasks[ti];
+    // LU: the tiles of both sides in one launch
+    int32_t        ti = xcd_task( blockIdx.x, gridDim.x );
+    const bool     u  = ti >= ntasks;
+    T *__restrict__ L = u ? L1 : L0;
+    const T *__restrict__ Linv = u ? Linv1 : Linv0;
+    uint64_t *stamps  = u ? stamps1 : stamps0;
+    ti -= u ? ntasks : 0;
+    const row_task t = tasks[ti];
     const uint64_t t_stamp = stamp_begin( stamps );
     wave_priority( prio );
     const dcblk    c    = cb[t.cblk];
