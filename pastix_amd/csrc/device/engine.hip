@@ -146,7 +146,7 @@ struct pxd_ctx_s {
 
     // matrix
     int      mflt = 0, mtx = 0;
-    int64_t  nnz = 0;
+    int64_t  nnz = 0, mat_n = 0;   // of the matrix buffers
     int64_t *dcolptr = nullptr, *drowtab = nullptr, *dtcolptr = nullptr, *dtrowtab = nullptr;
     void    *dval = nullptr, *dtval = nullptr;
     std::vector<int64_t> hcolptr, hrowtab;   // kept for the fill of the U side
@@ -332,14 +332,10 @@ template <> struct type_tag<float> { static constexpr int value = 1; };
 template <> struct type_tag<pxcd> { static constexpr int value = 2; };
 template <> struct type_tag<pxcf> { static constexpr int value = 3; };
 
-// Build the task lists of the factorization and the solve, level by level.
+// Whether the widest cblk fits the TRSM tiles (3: not); sets their rows.
 int
-build_schedule( pxd_ctx_t *ctx )
+check_width( pxd_ctx_t *ctx )
 {
-    const int64_t               nc    = ctx->cblknbr;
-    const std::vector<int32_t> &level = ctx->level;
-    const int32_t               nlev  = ctx->nlev;
-
     // the trsm tile keeps RT rows x n columns in LDS (static LDS of the kernel ~9 KB)
     if ( ctx->kernels ) {
         ctx->trsm_rt = 64;
@@ -356,6 +352,20 @@ build_schedule( pxd_ctx_t *ctx )
         fprintf( stderr, "pastix_amd device: cblk width %d exceeds the LDS budget of the TRSM tile\n",
                  ctx->colmax );
         return 3;
+    }
+    return 0;
+}
+
+// Build the task lists of the factorization and the solve, level by level.
+int
+build_schedule( pxd_ctx_t *ctx )
+{
+    const int64_t               nc    = ctx->cblknbr;
+    const std::vector<int32_t> &level = ctx->level;
+    const int32_t               nlev  = ctx->nlev;
+
+    if ( const int rc = check_width( ctx ) ) {
+        return rc;
     }
 
     // within a level, the cblks of the Schur part come after the others
@@ -806,8 +816,9 @@ factorize( pxd_ctx_t *ctx, double thresh, int64_t *nbpivots )
     double t_panel = 0., t_trsm = 0., t_upd = 0.;
     int64_t launches = 0;
 
-    PXD_CHECK( hipMemsetAsync( ctx->dscratch, 0, 4 * sizeof( int ), s ) );
-    PXD_CHECK( hipMemsetAsync( ctx->dflags, 0, sizeof( int ) * std::max<int64_t>( 1, ctx->npan ), s ) );
+    double *const dthresh = (double *)( ctx->dscratch + 8 );
+    hipLaunchKernelGGL( k_fact_begin, dim3( nblocks( std::max<int64_t>( 1, ctx->npan ), 256 ) ), dim3( 256 ), 0, s,
+                        ctx->dscratch, dthresh, thresh, ctx->dflags, ctx->npan );
     PXD_CHECK( hipEventRecord( e0, s ) );
 
     // fill: zero + scatter of the lower triangle of P A P^T (LU: and of the
@@ -908,17 +919,17 @@ factorize( pxd_ctx_t *ctx, double thresh, int64_t *nbpivots )
                 }
                 if ( lu ) {
                     hipLaunchKernelGGL( ( k_panel<T, PAN_LU> ), grid, dim3( PXD_THREADS ), 0, st, ctx->dpan + q0,
-                                        ctx->dcb, L, U, DI, DU, thresh, ctx->dscratch, ctx->dflags, ctx->dscratch + 2,
+                                        ctx->dcb, L, U, DI, DU, dthresh, ctx->dscratch, ctx->dflags, ctx->dscratch + 2,
                                         sp, ctx->prio );
                 }
                 else if ( ldlt ) {
                     hipLaunchKernelGGL( ( k_panel<T, PAN_LDLT> ), grid, dim3( PXD_THREADS ), 0, st, ctx->dpan + q0,
-                                        ctx->dcb, L, L, DI, DI, thresh, ctx->dscratch, ctx->dflags, ctx->dscratch + 2,
+                                        ctx->dcb, L, L, DI, DI, dthresh, ctx->dscratch, ctx->dflags, ctx->dscratch + 2,
                                         sp, ctx->prio );
                 }
                 else if constexpr ( std::is_same<T, R>::value ) {
                     hipLaunchKernelGGL( ( k_panel<T, PAN_LLT> ), grid, dim3( PXD_THREADS ), 0, st, ctx->dpan + q0,
-                                        ctx->dcb, L, L, DI, DI, thresh, ctx->dscratch, ctx->dflags, ctx->dscratch + 2,
+                                        ctx->dcb, L, L, DI, DI, dthresh, ctx->dscratch, ctx->dflags, ctx->dscratch + 2,
                                         sp, ctx->prio );
                 }
                 launches++;
@@ -1092,7 +1103,8 @@ factorize( pxd_ctx_t *ctx, double thresh, int64_t *nbpivots )
             // the level loop (both streams) as one graph, captured once per
             // structure and factor buffers; the clearing and the fill above
             // stay outside it
-            const fact_graph_sig sig{ type_tag<T>::value, ctx->sched_gen, L, U, DI, DU, thresh, ctx->prio,
+            // (k_panel reads the threshold from memory, the others have it baked in)
+            const fact_graph_sig sig{ type_tag<T>::value, ctx->sched_gen, L, U, DI, DU, use_mw ? 0. : thresh, ctx->prio,
                                       ctx->panel_mw, ldlt };
             if ( ctx->fgraph == nullptr || !( ctx->fgraph_sig == sig ) ) {
                 if ( ctx->fgraph ) {
@@ -2299,8 +2311,10 @@ pxd_set_structure( pxd_ctx_t *ctx, int64_t n, int64_t cblknbr, int64_t bloknbr,
         return 6;
     }
     compute_levels( ctx, cblks, bloks, browtab );
-    ctx->tasks_dirty = 0;
-    return build_schedule( ctx );
+    // the task lists follow with the first factorization, which says its kind
+    ctx->tasks_dirty  = 1;
+    ctx->stats.levels = ctx->nlev;
+    return check_width( ctx );
 }
 
 int
@@ -2315,26 +2329,34 @@ pxd_set_matrix( pxd_ctx_t *ctx, int flttype, int mtxtype, int64_t n, int64_t nnz
     if ( n != ctx->n ) {
         return 7;
     }
-    ctx->mflt = flttype;
-    ctx->mtx  = mtxtype;
-    ctx->nnz  = nnz;
-    size_t es = elt_size( flttype );
-    void *ptrs[] = { ctx->dcolptr, ctx->drowtab, ctx->dval, ctx->dtcolptr, ctx->dtrowtab, ctx->dtval };
-    for ( void *p : ptrs ) {
-        if ( p ) PXD_CHECK( hipFree( p ) );
+    const size_t es   = elt_size( flttype );
+    const size_t nnz1 = std::max<int64_t>( nnz, 1 );
+    // new values of the same pattern sizes go to the buffers that are there
+    if ( ctx->dval == nullptr || ctx->mat_n != n || ctx->nnz != nnz || ctx->mflt != flttype ||
+         ( ctx->dtval != nullptr ) != ( tcolptr != nullptr ) ) {
+        void **ptrs[] = { (void **)&ctx->dcolptr, (void **)&ctx->drowtab, &ctx->dval, (void **)&ctx->dtcolptr,
+                          (void **)&ctx->dtrowtab, &ctx->dtval };
+        for ( void **p : ptrs ) {
+            if ( *p ) PXD_CHECK( hipFree( *p ) );
+            *p = nullptr;
+        }
+        ctx->mflt  = flttype;
+        ctx->nnz   = nnz;
+        ctx->mat_n = n;
+        PXD_CHECK( hipMalloc( (void **)&ctx->dcolptr, ( n + 1 ) * sizeof( int64_t ) ) );
+        PXD_CHECK( hipMalloc( (void **)&ctx->drowtab, nnz1 * sizeof( int64_t ) ) );
+        if ( tcolptr ) {
+            PXD_CHECK( hipMalloc( (void **)&ctx->dtcolptr, ( n + 1 ) * sizeof( int64_t ) ) );
+            PXD_CHECK( hipMalloc( (void **)&ctx->dtrowtab, nnz1 * sizeof( int64_t ) ) );
+            PXD_CHECK( hipMalloc( &ctx->dtval, nnz1 * es ) );
+        }
+        PXD_CHECK( hipMalloc( &ctx->dval, nnz1 * es ) );   // last: dval says that all are there
     }
-    ctx->dcolptr = ctx->drowtab = ctx->dtcolptr = ctx->dtrowtab = nullptr;
-    ctx->dval = ctx->dtval = nullptr;
-    PXD_CHECK( hipMalloc( (void **)&ctx->dcolptr, ( n + 1 ) * sizeof( int64_t ) ) );
-    PXD_CHECK( hipMalloc( (void **)&ctx->drowtab, std::max<int64_t>( nnz, 1 ) * sizeof( int64_t ) ) );
-    PXD_CHECK( hipMalloc( &ctx->dval, std::max<int64_t>( nnz, 1 ) * es ) );
+    ctx->mtx = mtxtype;
     PXD_CHECK( hipMemcpy( ctx->dcolptr, colptr, ( n + 1 ) * sizeof( int64_t ), hipMemcpyHostToDevice ) );
     PXD_CHECK( hipMemcpy( ctx->drowtab, rowtab, nnz * sizeof( int64_t ), hipMemcpyHostToDevice ) );
     PXD_CHECK( hipMemcpy( ctx->dval, values, nnz * es, hipMemcpyHostToDevice ) );
     if ( tcolptr ) {
-        PXD_CHECK( hipMalloc( (void **)&ctx->dtcolptr, ( n + 1 ) * sizeof( int64_t ) ) );
-        PXD_CHECK( hipMalloc( (void **)&ctx->dtrowtab, std::max<int64_t>( nnz, 1 ) * sizeof( int64_t ) ) );
-        PXD_CHECK( hipMalloc( &ctx->dtval, std::max<int64_t>( nnz, 1 ) * es ) );
         PXD_CHECK( hipMemcpy( ctx->dtcolptr, tcolptr, ( n + 1 ) * sizeof( int64_t ), hipMemcpyHostToDevice ) );
         PXD_CHECK( hipMemcpy( ctx->dtrowtab, trowtab, nnz * sizeof( int64_t ), hipMemcpyHostToDevice ) );
         PXD_CHECK( hipMemcpy( ctx->dtval, tvalues, nnz * es, hipMemcpyHostToDevice ) );

@@ -49,6 +49,17 @@ struct pan_task {
 #define PXD_PAN_COL   ( 1 << 16 )
 #define PXD_PAN_USIDE ( 1 << 17 )
 
+// Start of a factorization: counters, the pivot threshold (in memory, so that a
+// captured factorization serves every matrix of the structure) and the flags.
+__global__ void
+k_fact_begin( int *scratch, double *dthresh, double thresh, int *flags, int64_t nflags )
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if ( i < nflags ) flags[i] = 0;
+    if ( i < 4 ) scratch[i] = 0;
+    if ( i == 0 ) *dthresh = thresh;
+}
+
 enum { PAN_LLT = 0, PAN_LDLT = 1, PAN_LU = 2 };
 
 // Bound of one wait in ticks of the constant clock (wall_clock64), set on
@@ -210,7 +221,8 @@ panel_inverse_column( const T *A, T *LI, int32_t n, int J, int nblk, const int *
 
 template <typename T, int KIND>
 __global__ void __launch_bounds__( PXD_THREADS )
-k_panel( const pan_task *__restrict__ tasks, const dcblk *__restrict__ cb, T *L, T *U, T *DL, T *DU, double thresh,
+k_panel( const pan_task *__restrict__ tasks, const dcblk *__restrict__ cb, T *L, T *U, T *DL, T *DU,
+         const double *__restrict__ thresh,
          int *__restrict__ npiv, int *flags, int *err, uint64_t *__restrict__ stamps, int prio )
 {
     typedef mfma16<T>                 M;
@@ -413,7 +425,7 @@ k_panel( const pan_task *__restrict__ tasks, const dcblk *__restrict__ cb, T *L,
         if constexpr ( LU ) sZ[cc][r] = ( r == cc && r < bs ) ? (T)1 : (T)0;
     }
     __syncthreads();
-    const R tau = (R)thresh;
+    const R tau = (R)*thresh;
     int     piv = 0;
     if ( w == 0 ) {
         piv = elim32<T, KIND != PAN_LLT, LU>( sA, sI, sZ, sD, bs, tau, lane );

@@ -568,6 +568,7 @@ pastix_subtask_blend( pastix_data_t *pd )
     else {
         pd->solvmatr = px_calloc( 1, sizeof( px_solver_t ) );
     }
+    pd->dev_structure = 0;
     px_solver_gen( pd->solvmatr, pd->symbmtx, pd->iparm[IPARM_TASKS2D_WIDTH], pd->iparm[IPARM_TASKS2D_LEVEL] );
     if ( px_solver_check( pd->solvmatr ) != PASTIX_SUCCESS ) {
         px_print_error( "pastix_subtask_blend: inconsistent solver matrix" );
@@ -627,6 +628,7 @@ px_device_ready( pastix_data_t *pd )
     if ( pd->dev != NULL ) {
         return PASTIX_SUCCESS;
     }
+    pd->dev_structure = 0;
     rc = pxd_create( &pd->dev, 0 );
     if ( rc != PASTIX_SUCCESS ) {
         pd->dev = NULL;
@@ -712,8 +714,13 @@ pastix_subtask_bcsc2ctab( pastix_data_t *pd )
     if ( ( rc = px_device_ready( pd ) ) != PASTIX_SUCCESS ) {
         return rc;
     }
-    if ( ( rc = px_upload_structure( pd ) ) != PASTIX_SUCCESS ) {
-        return rc;
+    /* once per analysis: later factorizations bring new values only, and the
+     * engine keeps its task lists and captured graphs */
+    if ( !pd->dev_structure ) {
+        if ( ( rc = px_upload_structure( pd ) ) != PASTIX_SUCCESS ) {
+            return rc;
+        }
+        pd->dev_structure = 1;
     }
     {
         px_bcsc_t *b = pd->bcsc;

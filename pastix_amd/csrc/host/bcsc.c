@@ -33,6 +33,25 @@ cmp_entry( const void *a, const void *b )
     return ( x > y ) - ( x < y );
 }
 
+/* By row: in place for the lengths of grid columns, whose qsort calls took
+ * most of a small matrix's numfact. */
+static void
+sort_entries( entry_t *t, pastix_int_t n )
+{
+    if ( n > 64 ) {
+        qsort( t, n, sizeof( entry_t ), cmp_entry );
+        return;
+    }
+    for ( pastix_int_t k = 1; k < n; k++ ) {
+        const entry_t x = t[k];
+        pastix_int_t  i = k;
+        for ( ; i > 0 && t[i - 1].r > x.r; i-- ) {
+            t[i] = t[i - 1];
+        }
+        t[i] = x;
+    }
+}
+
 /* Build a CSC from (row, col, value) triplets, summing duplicates. */
 static void
 build_csc( pastix_int_t n, pastix_int_t ne, const pastix_int_t *ri, const pastix_int_t *ci,
@@ -65,7 +84,7 @@ build_csc( pastix_int_t n, pastix_int_t ne, const pastix_int_t *ri, const pastix
     ptr[0] = 0;
     for ( pastix_int_t j = 0; j < n; j++ ) {
         pastix_int_t b = cnt[j], e = cnt[j + 1];
-        qsort( tmp + b, e - b, sizeof( entry_t ), cmp_entry );
+        sort_entries( tmp + b, e - b );
         for ( pastix_int_t k = b; k < e; k++ ) {
             if ( nnz > ptr[j] && rows[nnz - 1] == tmp[k].r ) {
                 if ( cplx ) {

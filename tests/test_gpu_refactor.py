@@ -1,0 +1,77 @@
+"""Several numerical factorizations of one analysed structure: the engine keeps
+the structure, its task lists and its captured graphs, and takes the new
+values, norms and pivot thresholds, another factorization and precision, and
+a new analysis.  Every factor against the oracle, every solve by its backward
+error."""
+import numpy as np
+import pytest
+
+import pastix_amd as px
+import oracle_ref as orc
+from helpers import analyzed, cblk_diff, make_problem, static_pivot_threshold
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(pd, iparm, dparm, spm, facto, mixed):
+    iparm[px.IPARM_FACTORIZATION] = facto
+    iparm[px.IPARM_MIXED] = mixed
+    px.task_numfact(pd, spm)
+    dtype = np.float32 if mixed else np.float64
+    s = px.solver_export(pd)
+    oracle = {px.PastixFactPOTRF: orc.OracleFactor, px.PastixFactLDLT: orc.OracleLDLT, px.PastixFactLU: orc.OracleLU}
+    F = oracle[facto](s, px.bcsc_export(pd), static_pivot_threshold(dparm, dtype), dtype)
+    assert iparm[px.IPARM_STATIC_PIVOTING] == F.npiv
+    assert cblk_diff(s, px.get_coeftab(pd, s["coefnbr"], dtype), F.L, dtype, full_diag=facto != px.PastixFactPOTRF) <= 10.0
+    x0, b = spm.gen_rhs(3, seed=1)
+    x = np.array(b, order="F", copy=True)
+    px.task_solve(pd, spm, x)
+    assert spm.backward_error(b, x)[0] <= (1e-5 if mixed else 1e-14)
+
+
+def test_new_values_kinds_and_precisions_on_one_structure():
+    nx = 13
+    base = make_problem("lap7", nx)
+    cp, rp, v = base.arrays()
+    rng = np.random.default_rng(3)
+    first = px.Spm.from_csc(nx ** 3, cp, rp, v, mtxtype=base.s.mtxtype)
+    pd, iparm, dparm = analyzed(first, nx)
+    mats = [first]
+    for scale in (1e3, 1e-4, 1.0):   # thresholds follow the norm
+        w = v * scale * (1.0 + 0.1 * rng.random(v.shape))
+        mats.append(px.Spm.from_csc(nx ** 3, cp, rp, w, mtxtype=base.s.mtxtype))
+    for facto, mixed in [(px.PastixFactPOTRF, 0), (px.PastixFactLDLT, 0), (px.PastixFactPOTRF, 1), (px.PastixFactLU, 0),
+                         (px.PastixFactPOTRF, 0)]:
+        for m in mats:
+            _check(pd, iparm, dparm, m, facto, mixed)
+    # a new analysis on the same instance
+    other = make_problem("lap7", nx)
+    px.analyze_grid(pd, other, nx, nx, nx)
+    _check(pd, iparm, dparm, other, px.PastixFactPOTRF, 0)
+    smaller = make_problem("lap7", nx - 3)
+    px.analyze_grid(pd, smaller, nx - 3, nx - 3, nx - 3)
+    _check(pd, iparm, dparm, smaller, px.PastixFactPOTRF, 0)
+    px.finalize(pd)
+
+
+def test_threshold_of_a_captured_factorization_follows_the_matrix():
+    """A zero pivot is replaced by the threshold of its own matrix: the same
+    structure with the values scaled by 1e6 in between."""
+    nx = 6
+    base = make_problem("lap7", nx)
+    cp, rp, v = base.arrays()
+    v = v.copy()
+    for j in (5, 77):   # unknowns cut off, with a zero diagonal
+        for c in range(nx ** 3):
+            for p in range(cp[c], cp[c + 1]):
+                if c == j or rp[p] == j:
+                    v[p] = 0.0
+    spms = [px.Spm.from_csc(nx ** 3, cp, rp, v * f, mtxtype=base.s.mtxtype) for f in (1.0, 1e6, 1.0)]
+    pd, iparm, dparm = analyzed(spms[0], nx)
+    for m in spms:
+        px.task_numfact(pd, m)
+        s = px.solver_export(pd)
+        F = orc.OracleFactor(s, px.bcsc_export(pd), static_pivot_threshold(dparm, np.float64))
+        assert iparm[px.IPARM_STATIC_PIVOTING] == F.npiv == 2
+        assert cblk_diff(s, px.get_coeftab(pd, s["coefnbr"], np.float64), F.L, np.float64) <= 10.0
+    px.finalize(pd)
