@@ -1687,19 +1687,24 @@ wide_pass( pxd_ctx_t *ctx, TV *v, int64_t ld, int nq, bool swap )
 }
 
 // Fewest right-hand sides for which a wide pass is the faster one (measured,
-// narrow against wide): in double always (100^3: 5.80 against 5.22 ms for 1
-// and 9.7 against 5.8 ms for 8; 41^3 LU 0.59 / 0.51 ms for 1); in single from
-// 5 on (100^3: 4.14 against 4.92 ms for 4, 5.48 against 4.80 ms for 5), and on
-// small systems, which are all latency, always (25^3: 0.23 against 0.16 ms
-// for 4; 50^3, 125,000 unknowns: 0.698 against 0.701 ms).
+// narrow against wide, ms): in double always (100^3: 5.80 / 5.22 for 1 and
+// 9.7 / 5.8 for 8; 41^3 LU 0.59 / 0.51 for 1; 15^3 complex 0.154 / 0.142); in
+// single from 5 on (100^3: 4.14 / 4.92 for 4, 5.48 / 4.80 for 5), and always on
+// small factors, which are all latency: real ones (40^3, 95 MB: 0.455 / 0.436
+// for 1; 50^3, 245 MB: 0.698 / 0.701 for 4; 41^3 LU, 235 MB: 0.484 / 0.509 for
+// 1), and complex ones, four products for each, only while they are tiny (15^3,
+// 3 MB: 0.136 / 0.127 for 1; 25^3, 27 MB: 0.239 / 0.265).
 template <typename T>
 int64_t
 wide_from( const pxd_ctx_t *ctx )
 {
+    typedef typename px_real<T>::type R;
     if ( ctx->solve_wide_rhs > 0 ) {
         return ctx->solve_wide_rhs;
     }
-    return sizeof( typename px_real<T>::type ) == 8 || ctx->n < 100000 ? 1 : 5;
+    const int64_t small = ( sizeof( T ) > sizeof( R ) ) ? 4 << 20 : 100 << 20;
+    const int64_t bytes = (int64_t)sizeof( T ) * ctx->coefnbr * ( ctx->facto == FACT_GETRF ? 2 : 1 );
+    return sizeof( R ) == 8 || bytes < small ? 1 : 5;
 }
 
 template <typename TV, typename T>
