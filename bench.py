@@ -487,7 +487,7 @@ def main():
                      "unit": "TFLOP/s", "frac": achieved / MFMA_PEAK_TFLOPS["f32"], "traffic": traffic,
                      "traffic_scope": "HBM bytes of the update launches of one factorization (rocprofv3 FETCH_SIZE "
                                       "+ WRITE_SIZE, copy-calibrated)", "traffic_per_launch": traffic_launch,
-                     "kernel": "k_update_dma<8,3> + k_update_mfma<float> + k_update_small<float> (supernodal "
+                     "kernel": "k_update_dma<float> + k_update_mfma<float> + k_update_small<float> (supernodal "
                                "update, all launches of one factorization)", "algorithmic_flops": upd},
         "cpu_baseline": None,
     }
@@ -500,7 +500,7 @@ def main():
         a64, u64 = update_roofline(r64, "f64")
         out["roofline_fp64"] = {"bound": "mfma", "achieved": a64, "peak": MFMA_PEAK_TFLOPS["f64"], "unit": "TFLOP/s",
                                 "frac": a64 / MFMA_PEAK_TFLOPS["f64"], "traffic": traffic64,
-                                "kernel": "k_update_big<double> + k_update_mfma<double> + k_update_small<double> "
+                                "kernel": "k_update_dma<double> + k_update_mfma<double> + k_update_small<double> "
                                           "(all launches of one factorization)", "algorithmic_flops": u64}
         out["roofline_solve_fp64"] = r64["bandwidth"]["solve"]
         # forward error of the FP32+IR solution against the FP64 factorization's

@@ -84,7 +84,8 @@ int  pxd_get_stats( const pxd_ctx_t *ctx, pxd_stats_t *stats );
  *   "timing"        1: one stream, per-phase kernel times in the stats
  *   "model_log"     1: kernel timing log of the next factorization
  *   "kernels"       1: matrix-core kernels (default); 0: scalar kernels
- *   "panel_mw"      1: multi-workgroup Cholesky panels (default)
+ *   "panel_mw"      1: multi-workgroup panels (default); 0: Cholesky panels
+ *                   by one workgroup per cblk
  *   "upd_big_rows"  stacked rows from which updates use the tall tiles
  *   "upd_small"     1: one-wavefront small updates (default)
  *   "upd_small_m", "upd_small_n"  largest stacked rows (up to 256, default
@@ -102,6 +103,10 @@ int  pxd_get_stats( const pxd_ctx_t *ctx, pxd_stats_t *stats );
  *                   graph captured on first use (default); 0: launched one by one
  *   "solve_wide_max" level-solve launches with at least this many tiles load
  *                   16 columns per batch (default 128)
+ *   "solve_wide_rhs" fewest right-hand sides that a solve takes in blocks of
+ *                   4, 16 or 32 on the matrix cores; 0 (default): the
+ *                   measured rule (double: 1; single: 5, fewer on small
+ *                   systems)
  *   "solve_small"   1: levels of cblks of at most 16 columns solve with one
  *                   wavefront per cblk, one launch per level (default)
  *   "solve_spread"  cblks with at least this many 64-row tiles (default 16;

@@ -13,7 +13,7 @@ rounding:
   values;
 - ``solve_wide_max``: level-solve launches from which the tiles load 16
   columns per batch instead of all of them;
-- ``panel_mw``: the multi-workgroup Cholesky panel;
+- ``panel_mw``: the multi-workgroup panel (0: Cholesky by one workgroup);
 - ``upd_dma``: tall tiles on the kernel that loads its operands straight
   into LDS;
 - ``upd_dma_pad``: extra LDS per workgroup of that kernel, which sets how
