@@ -2316,6 +2316,11 @@ pxd_set_structure( pxd_ctx_t *ctx, int64_t n, int64_t cblknbr, int64_t bloknbr,
         return 6;
     }
     compute_levels( ctx, cblks, bloks, browtab );
+    if ( ctx->dL != nullptr ) {
+        // a factor is there to solve with, whose lists belong to the structure
+        ctx->tasks_dirty = 0;
+        return build_schedule( ctx );
+    }
     // the task lists follow with the first factorization, which says its kind
     ctx->tasks_dirty  = 1;
     ctx->stats.levels = ctx->nlev;
@@ -2356,6 +2361,10 @@ pxd_set_matrix( pxd_ctx_t *ctx, int flttype, int mtxtype, int64_t n, int64_t nnz
             PXD_CHECK( hipMalloc( &ctx->dtval, nnz1 * es ) );
         }
         PXD_CHECK( hipMalloc( &ctx->dval, nnz1 * es ) );   // last: dval says that all are there
+    }
+    else {
+        // products with the old values that are still in flight (hipFree waits)
+        PXD_CHECK( hipStreamSynchronize( ctx->stream ) );
     }
     ctx->mtx = mtxtype;
     PXD_CHECK( hipMemcpy( ctx->dcolptr, colptr, ( n + 1 ) * sizeof( int64_t ), hipMemcpyHostToDevice ) );

@@ -3,6 +3,8 @@ the structure, its task lists and its captured graphs, and takes the new
 values, norms and pivot thresholds, another factorization and precision, and
 a new analysis.  Every factor against the oracle, every solve by its backward
 error."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -74,4 +76,40 @@ def test_threshold_of_a_captured_factorization_follows_the_matrix():
         F = orc.OracleFactor(s, px.bcsc_export(pd), static_pivot_threshold(dparm, np.float64))
         assert iparm[px.IPARM_STATIC_PIVOTING] == F.npiv == 2
         assert cblk_diff(s, px.get_coeftab(pd, s["coefnbr"], np.float64), F.L, np.float64) <= 10.0
+    px.finalize(pd)
+
+
+def test_products_in_flight_take_the_old_values():
+    """New values reach the same buffers: products issued before they came
+    use the old ones."""
+    nx, nrhs, scale = 40, 8, 2.0
+    n = nx ** 3
+    base = make_problem("lap7", nx)
+    cp, rp, v = base.arrays()
+    spms = [px.Spm.from_csc(n, cp, rp, v * f, mtxtype=base.s.mtxtype) for f in (1.0, scale)]
+    pd, iparm, dparm = analyzed(spms[0], nx)
+    px._check("spm2bcsc", px.lib.pastix_subtask_spm2bcsc(pd, ctypes.byref(spms[0].s)))
+    px._check("bcsc2ctab", px.lib.pastix_subtask_bcsc2ctab(pd))
+    px._check("spm2bcsc", px.lib.pastix_subtask_spm2bcsc(pd, ctypes.byref(spms[1].s)))
+    dev = ctypes.c_void_p()
+    px._check("device_handle", px.lib.pastix_amd_device_handle(pd, ctypes.byref(dev)))
+    x = np.ones(n * nrhs)
+    bufs = []
+    for k in range(22):   # the vectors, 20 products, the product with the new values
+        p = ctypes.c_void_p()
+        px._check("malloc", px.lib.pxd_malloc(dev, x.nbytes, ctypes.byref(p)))
+        px._check("h2d", px.lib.pxd_h2d(dev, p, x.ctypes.data_as(ctypes.c_void_p), x.nbytes))
+        bufs.append(p)
+    for y in bufs[1:21]:
+        px._check("pxd_spmv", px.lib.pxd_spmv(dev, 1.0, bufs[0], 0.0, y, nrhs, n))
+    px._check("bcsc2ctab", px.lib.pastix_subtask_bcsc2ctab(pd))
+    px._check("pxd_spmv", px.lib.pxd_spmv(dev, 1.0, bufs[0], 0.0, bufs[21], nrhs, n))
+    out = []
+    for y in bufs[1:]:
+        out.append(np.zeros_like(x))
+        px._check("d2h", px.lib.pxd_d2h(dev, out[-1].ctypes.data_as(ctypes.c_void_p), y, x.nbytes))
+    for p in bufs:
+        px.lib.pxd_free(dev, p)
+    for y in out[:20]:
+        assert np.array_equal(scale * y, out[20])   # a power of two: exact
     px.finalize(pd)
