@@ -112,7 +112,9 @@ struct pxd_ctx_s {
     // schedule
     std::vector<int32_t> level;     // dependency level of each cblk
     int32_t              nlev = 0;
-    int                  tasks_dirty = 0;   // options changed the task lists
+    int                  tasks_dirty = 0;   // the task lists do not fit the structure, options and factorization
+    bool                 lists_ok    = false;   // the lists on the device are whole
+    bool                 structure_ok = false;  // ... and the structure
     std::vector<level_t> levels;
     int32_t  *dlist = nullptr;
     pan_task *dpan  = nullptr;
@@ -357,6 +359,9 @@ check_width( pxd_ctx_t *ctx )
 }
 
 // Build the task lists of the factorization and the solve, level by level.
+// They count as missing until all are there: a build that ends early leaves
+// tasks_dirty set, so that the next factorization builds them again, and no
+// graph captured on lists that are gone.
 int
 build_schedule( pxd_ctx_t *ctx )
 {
@@ -364,8 +369,16 @@ build_schedule( pxd_ctx_t *ctx )
     const std::vector<int32_t> &level = ctx->level;
     const int32_t               nlev  = ctx->nlev;
 
+    ctx->tasks_dirty = 1;
     if ( const int rc = check_width( ctx ) ) {
         return rc;
+    }
+    ctx->lists_ok = false;
+    ctx->sched_gen++;
+    drop_solve_graphs( ctx );
+    if ( ctx->fgraph ) {
+        (void)hipGraphExecDestroy( ctx->fgraph );
+        ctx->fgraph = nullptr;
     }
 
     // within a level, the cblks of the Schur part come after the others
@@ -674,8 +687,8 @@ build_schedule( pxd_ctx_t *ctx )
             return 6;
         }
     }
-    ctx->sched_gen++;
-    drop_solve_graphs( ctx );
+    ctx->tasks_dirty = 0;
+    ctx->lists_ok    = true;
     return 0;
 }
 
@@ -1795,7 +1808,7 @@ int
 solve_steps( pxd_ctx_t *ctx, int what, bool swap, int64_t nrhs, void *dx, int64_t ldx )
 {
     PXD_CHECK( hipSetDevice( ctx->device ) );
-    if ( ctx->dL == nullptr || nrhs < 0 || ( nrhs > 0 && ( dx == nullptr || ldx < ctx->n ) ) ) {
+    if ( ctx->dL == nullptr || !ctx->lists_ok || nrhs < 0 || ( nrhs > 0 && ( dx == nullptr || ldx < ctx->n ) ) ) {
         return 7;
     }
     if ( nrhs == 0 || ctx->n == 0 ) {
@@ -2258,6 +2271,10 @@ pxd_set_structure( pxd_ctx_t *ctx, int64_t n, int64_t cblknbr, int64_t bloknbr,
         return 3;
     }
     PXD_CHECK( hipSetDevice( ctx->device ) );
+    // an upload that ends early leaves nothing to factorize or solve with
+    ctx->structure_ok = false;
+    ctx->lists_ok     = false;
+    ctx->tasks_dirty  = 1;
     ctx->n       = n;
     ctx->schurfcol = n;   // no Schur part until pxd_set_schur
     ctx->cblknbr = cblknbr;
@@ -2316,13 +2333,12 @@ pxd_set_structure( pxd_ctx_t *ctx, int64_t n, int64_t cblknbr, int64_t bloknbr,
         return 6;
     }
     compute_levels( ctx, cblks, bloks, browtab );
+    ctx->structure_ok = true;
     if ( ctx->dL != nullptr ) {
         // a factor is there to solve with, whose lists belong to the structure
-        ctx->tasks_dirty = 0;
         return build_schedule( ctx );
     }
     // the task lists follow with the first factorization, which says its kind
-    ctx->tasks_dirty  = 1;
     ctx->stats.levels = ctx->nlev;
     return check_width( ctx );
 }
@@ -2406,7 +2422,7 @@ int
 pxd_factorize( pxd_ctx_t *ctx, int factotype, int factor_flttype, double threshold, int64_t *nbpivots )
 {
     PXD_CHECK( hipSetDevice( ctx->device ) );
-    if ( ctx->dval == nullptr || ctx->dcb == nullptr ) {
+    if ( ctx->dval == nullptr || !ctx->structure_ok ) {
         return 7;
     }
     if ( factotype != FACT_POTRF && factotype != FACT_GETRF && factotype != FACT_SYTRF ) {
@@ -2456,11 +2472,13 @@ pxd_factorize( pxd_ctx_t *ctx, int factotype, int factor_flttype, double thresho
                  : ( factor_flttype == FT_FLOAT ) ? upd_rows<float>::value
                  : ( factor_flttype == FT_CPLX64 ) ? upd_rows<pxcd>::value : upd_rows<pxcf>::value;
     if ( ctx->tasks_dirty || ctx->upd_bm != bm || ctx->facto != factotype ) {
-        ctx->upd_bm      = bm;
-        ctx->facto       = factotype;
-        ctx->tasks_dirty = 0;
+        const bool same = ( ctx->facto == factotype );
+        ctx->upd_bm = bm;
+        ctx->facto  = factotype;
         int rc = build_schedule( ctx );
         if ( rc ) {
+            // lists left from another factorization fit no factor of this kind
+            ctx->lists_ok = ctx->lists_ok && same;
             return rc;
         }
     }
@@ -2507,7 +2525,7 @@ int
 pxd_solve_noalloc( pxd_ctx_t *ctx, int64_t nrhs, void *dx, int64_t ldx )
 {
     PXD_CHECK( hipSetDevice( ctx->device ) );
-    if ( ctx->dL == nullptr || nrhs < 0 || ( nrhs > 0 && ( dx == nullptr || ldx < ctx->n ) ) ) {
+    if ( ctx->dL == nullptr || !ctx->lists_ok || nrhs < 0 || ( nrhs > 0 && ( dx == nullptr || ldx < ctx->n ) ) ) {
         return 7;
     }
     if ( nrhs == 0 || ctx->n == 0 ) {
@@ -2568,7 +2586,7 @@ int
 pxd_get_diag( pxd_ctx_t *ctx, void *dd )
 {
     PXD_CHECK( hipSetDevice( ctx->device ) );
-    if ( ctx->dL == nullptr || dd == nullptr ) {
+    if ( ctx->dL == nullptr || !ctx->structure_ok || dd == nullptr ) {
         return 7;
     }
     const unsigned nb = nblocks( ctx->n, 256 );

@@ -2,7 +2,8 @@
 the structure, its task lists and its captured graphs, and takes the new
 values, norms and pivot thresholds, another factorization and precision, and
 a new analysis.  Every factor against the oracle, every solve by its backward
-error."""
+error.  A factorization whose task lists cannot be built says so every time
+and leaves nothing behind that a later one would run on."""
 import ctypes
 
 import numpy as np
@@ -112,4 +113,27 @@ def test_products_in_flight_take_the_old_values():
         px.lib.pxd_free(dev, p)
     for y in out[:20]:
         assert np.array_equal(scale * y, out[20])   # a power of two: exact
+    px.finalize(pd)
+
+
+def test_lists_that_cannot_be_built_are_refused_every_time():
+    """A cblk of 360 columns fits the scalar kernels and not the 352 columns
+    of the matrix-core TRSM, whose row tiles are of another height: the lists
+    of one are no lists for the other."""
+    nx, ny = 363, 360
+    spm = make_problem("lap7", nx, ny, 1)
+    pd, iparm, dparm = analyzed(spm, nx, ny, 1, extra={px.IPARM_MIN_BLOCKSIZE: 400, px.IPARM_MAX_BLOCKSIZE: 400})
+    s = px.solver_export(pd)
+    cb = s["cblk"].reshape(-1, 6)[:s["cblknbr"]]
+    assert (cb[:, 1] - cb[:, 0] + 1).max() == 360
+    for kernels, ok in ((0, True), (1, False), (1, False), (0, True)):
+        px.set_option(pd, "kernels", kernels)
+        if not ok:
+            with pytest.raises(px.PastixError) as e:
+                px.task_numfact(pd, spm)
+            assert e.value.code == px.PASTIX_ERR_NOTIMPLEMENTED
+            continue
+        px.task_numfact(pd, spm)
+        F = orc.OracleFactor(s, px.bcsc_export(pd), static_pivot_threshold(dparm, np.float64))
+        assert cblk_diff(s, px.get_coeftab(pd, s["coefnbr"], np.float64), F.L, np.float64) <= 10.0
     px.finalize(pd)
