@@ -140,6 +140,9 @@ int  pxd_d2h    ( pxd_ctx_t *ctx, void *dst, const void *src, size_t bytes );
 int pxd_set_structure( pxd_ctx_t *ctx, int64_t n, int64_t cblknbr, int64_t bloknbr,
                        const pxd_cblk_t *cblks, const pxd_blok_t *bloks,
                        const int64_t *browtab, int64_t coefnbr );
+/* Structures uploaded to the context so far (a caller that keeps one there
+ * knows by it whether another has come since). */
+int64_t pxd_structure_count( const pxd_ctx_t *ctx );
 
 /*
  * Schur complement (reference sopalin/schur.c, blend's CBLK_IN_SCHUR): the

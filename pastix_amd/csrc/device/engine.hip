@@ -115,6 +115,7 @@ struct pxd_ctx_s {
     int                  tasks_dirty = 0;   // the task lists do not fit the structure, options and factorization
     bool                 lists_ok    = false;   // the lists on the device are whole
     bool                 structure_ok = false;  // ... and the structure
+    int64_t              structures  = 0;       // pxd_set_structure calls
     std::vector<level_t> levels;
     int32_t  *dlist = nullptr;
     pan_task *dpan  = nullptr;
@@ -2271,6 +2272,7 @@ pxd_set_structure( pxd_ctx_t *ctx, int64_t n, int64_t cblknbr, int64_t bloknbr,
         return 3;
     }
     PXD_CHECK( hipSetDevice( ctx->device ) );
+    ctx->structures++;
     // an upload that ends early leaves nothing to factorize or solve with
     ctx->structure_ok = false;
     ctx->lists_ok     = false;
@@ -2341,6 +2343,12 @@ pxd_set_structure( pxd_ctx_t *ctx, int64_t n, int64_t cblknbr, int64_t bloknbr,
     // the task lists follow with the first factorization, which says its kind
     ctx->stats.levels = ctx->nlev;
     return check_width( ctx );
+}
+
+int64_t
+pxd_structure_count( const pxd_ctx_t *ctx )
+{
+    return ctx->structures;
 }
 
 int

@@ -715,12 +715,14 @@ pastix_subtask_bcsc2ctab( pastix_data_t *pd )
         return rc;
     }
     /* once per analysis: later factorizations bring new values only, and the
-     * engine keeps its task lists and captured graphs */
-    if ( !pd->dev_structure ) {
+     * engine keeps its task lists and captured graphs.  Again when a program
+     * has given the engine another structure through its handle. */
+    if ( pd->dev_structure == 0 || pd->dev_structure != pxd_structure_count( pd->dev ) ) {
+        pd->dev_structure = 0;
         if ( ( rc = px_upload_structure( pd ) ) != PASTIX_SUCCESS ) {
             return rc;
         }
-        pd->dev_structure = 1;
+        pd->dev_structure = pxd_structure_count( pd->dev );
     }
     {
         px_bcsc_t *b = pd->bcsc;

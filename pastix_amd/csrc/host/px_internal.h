@@ -190,7 +190,7 @@ struct pastix_data_s {
     px_solver_t     *solvmatr;
     px_bcsc_t       *bcsc;
     pxd_ctx_t       *dev;       /* device engine context (NULL until first use) */
-    int              dev_structure;      /* 1: dev holds solvmatr's structure (0 after blend) */
+    int64_t          dev_structure;      /* pxd_structure_count of solvmatr's upload (0: none since blend) */
     int              factored_flttype;   /* precision of the device factor    */
     int              nthreads;
     char            *dir_global;

@@ -137,3 +137,27 @@ def test_lists_that_cannot_be_built_are_refused_every_time():
         F = orc.OracleFactor(s, px.bcsc_export(pd), static_pivot_threshold(dparm, np.float64))
         assert cblk_diff(s, px.get_coeftab(pd, s["coefnbr"], np.float64), F.L, np.float64) <= 10.0
     px.finalize(pd)
+
+
+def test_structure_given_through_the_handle_is_replaced():
+    """A program that uses the engine under an instance with a structure of
+    its own (here that of narrower cblks): the instance's next factorization
+    runs on the instance's structure again."""
+    nx = 12
+    spm = make_problem("lap7", nx)
+    pd, iparm, dparm = analyzed(spm, nx)
+    _check(pd, iparm, dparm, spm, px.PastixFactPOTRF, 0)
+    other, _, _ = analyzed(spm, nx, extra={px.IPARM_MIN_BLOCKSIZE: 20, px.IPARM_MAX_BLOCKSIZE: 40})
+    s = px.solver_export(other)
+    assert s["cblknbr"] != px.solver_export(pd)["cblknbr"]
+    dev = ctypes.c_void_p()
+    px._check("device_handle", px.lib.pastix_amd_device_handle(pd, ctypes.byref(dev)))
+    blok = np.concatenate([s["blok"], np.zeros(5, dtype=np.int64)])   # and the final entry
+    f = px.lib.pxd_set_structure
+    f.argtypes = [ctypes.c_void_p] + [px.pastix_int] * 3 + [ctypes.c_void_p] * 3 + [px.pastix_int]
+    for _ in range(2):
+        px._check("pxd_set_structure", f(dev, nx ** 3, s["cblknbr"], s["bloknbr"], s["cblk"].ctypes.data,
+                                         blok.ctypes.data, s["browtab"].ctypes.data, s["coefnbr"]))
+        _check(pd, iparm, dparm, spm, px.PastixFactPOTRF, 0)
+    px.finalize(other)
+    px.finalize(pd)
