@@ -107,6 +107,10 @@ int  pxd_get_stats( const pxd_ctx_t *ctx, pxd_stats_t *stats );
  *                   4, 16 or 32 on the matrix cores; 0 (default): the
  *                   measured rule (double: 1; single: 5, fewer on small
  *                   systems)
+ *   "solve_wide_mb" most MiB of scratch of those blocks (n x 4, 16 or 32
+ *                   values, twice); 0 (default): what the device has.  A block
+ *                   that does not fit is taken narrower.  Setting it gives the
+ *                   scratch held so far back
  *   "solve_small"   1: levels of cblks of at most 16 columns solve with one
  *                   wavefront per cblk, one launch per level (default)
  *   "solve_spread"  cblks with at least this many 64-row tiles (default 16;

@@ -140,6 +140,8 @@ struct pxd_ctx_s {
     // fewest right-hand sides that a wide pass takes (kernels_svwide.hpp); 0:
     // the rule of wide_from()
     int       solve_wide_rhs = 0;
+    double    solve_wide_mb  = 0.;         // most MiB of a wide pass's scratch; 0: what the device has
+    size_t    wide_refused   = SIZE_MAX;   // bytes of a vector that the device had not got (since the factorization)
     // 1: levels of cblks of at most PXD_DIAG_ROWS columns solve with one
     // wavefront per cblk (diagonal and off-diagonal rows in one launch)
     int       solve_small = 1;
@@ -278,6 +280,37 @@ upload( T **d, const std::vector<T> &h )
         PXD_CHECK( hipMemcpy( *d, h.data(), h.size() * sizeof( T ), hipMemcpyHostToDevice ) );
     }
     return 0;
+}
+
+// At least need bytes at *d, which holds *bytes (its contents may go); 6 and
+// nothing at *d where the device has not got them.
+int
+grow( void **d, size_t *bytes, size_t need )
+{
+    if ( *bytes >= need ) {
+        return 0;
+    }
+    if ( *d ) {
+        PXD_CHECK( hipFree( *d ) );
+    }
+    *d     = nullptr;
+    *bytes = 0;
+    if ( hipMalloc( d, need ) != hipSuccess ) {
+        (void)hipGetLastError();
+        *d = nullptr;
+        return 6;
+    }
+    *bytes = need;
+    return 0;
+}
+int
+grow_or_say( void **d, size_t *bytes, size_t need )
+{
+    const int rc = grow( d, bytes, need );
+    if ( rc ) {
+        fprintf( stderr, "pastix_amd device: no %zu bytes for a solve's scratch\n", need );
+    }
+    return rc;
 }
 
 inline unsigned
@@ -1331,10 +1364,8 @@ solve_sweeps( pxd_ctx_t *ctx, V *X, int64_t ldx, int nrhs, int what = SOLVE_ALL,
         // the caller hands over (n x nrhs entries)
         if ( Yscr == nullptr ) {
             size_t need = (size_t)ctx->n * PXD_MAXRHS * sizeof( V );
-            if ( ctx->dsolvy_bytes < need ) {
-                if ( ctx->dsolvy ) PXD_CHECK( hipFree( ctx->dsolvy ) );
-                PXD_CHECK( hipMalloc( &ctx->dsolvy, need ) );
-                ctx->dsolvy_bytes = need;
+            if ( const int rc = grow_or_say( &ctx->dsolvy, &ctx->dsolvy_bytes, need ) ) {
+                return rc;
             }
         }
         V            *Y   = Yscr ? Yscr : (V *)ctx->dsolvy;
@@ -1345,10 +1376,8 @@ solve_sweeps( pxd_ctx_t *ctx, V *X, int64_t ldx, int nrhs, int what = SOLVE_ALL,
         const bool sp_ok = nrhs <= 4 ? sv_spread_ok<V, 4>::value : sv_spread_ok<V, PXD_MAXRHS>::value;
         if ( Yscr == nullptr && ctx->solve_spread && ctx->spread_cols > 0 && sp_ok ) {
             const size_t sneed = (size_t)PXD_SV_SPREAD * PXD_MAXRHS * ctx->spread_cols * sizeof( V );
-            if ( ctx->dspread_bytes < sneed ) {
-                if ( ctx->dspread ) PXD_CHECK( hipFree( ctx->dspread ) );
-                PXD_CHECK( hipMalloc( &ctx->dspread, sneed ) );
-                ctx->dspread_bytes = sneed;
+            if ( const int rc = grow_or_say( &ctx->dspread, &ctx->dspread_bytes, sneed ) ) {
+                return rc;
             }
             S = (V *)ctx->dspread;
         }
@@ -1538,22 +1567,13 @@ int
 graph_buffers( pxd_ctx_t *ctx )
 {
     const size_t need = (size_t)ctx->n * PXD_MAXRHS * sizeof( T );
-    if ( ctx->dvecs_bytes < need ) {
-        if ( ctx->dvecs ) PXD_CHECK( hipFree( ctx->dvecs ) );
-        PXD_CHECK( hipMalloc( &ctx->dvecs, need ) );
-        ctx->dvecs_bytes = need;
-    }
-    if ( ctx->dsolvy_bytes < need ) {
-        if ( ctx->dsolvy ) PXD_CHECK( hipFree( ctx->dsolvy ) );
-        PXD_CHECK( hipMalloc( &ctx->dsolvy, need ) );
-        ctx->dsolvy_bytes = need;
+    if ( grow_or_say( &ctx->dvecs, &ctx->dvecs_bytes, need ) || grow_or_say( &ctx->dsolvy, &ctx->dsolvy_bytes, need ) ) {
+        return 6;
     }
     // the backward partial sums, so that no allocation happens under capture
     const size_t sneed = (size_t)PXD_SV_SPREAD * PXD_MAXRHS * ctx->spread_cols * sizeof( T );
-    if ( sv_spread_ok<T, 4>::value && ctx->solve_spread && ctx->dspread_bytes < sneed ) {
-        if ( ctx->dspread ) PXD_CHECK( hipFree( ctx->dspread ) );
-        PXD_CHECK( hipMalloc( &ctx->dspread, sneed ) );
-        ctx->dspread_bytes = sneed;
+    if ( sv_spread_ok<T, 4>::value && ctx->solve_spread ) {
+        return grow_or_say( &ctx->dspread, &ctx->dspread_bytes, sneed );
     }
     return 0;
 }
@@ -1670,26 +1690,42 @@ wide_sweeps( pxd_ctx_t *ctx, T *X, T *Y, int nq, bool swap )
     return 0;
 }
 
-// One wide pass: nq <= NR columns of v.
+// The vectors' scratch is given back (the graphs hold its addresses).
+void
+drop_vectors( pxd_ctx_t *ctx )
+{
+    drop_solve_graphs( ctx );
+    if ( ctx->dvecs ) (void)hipFree( ctx->dvecs );
+    if ( ctx->dsolvy ) (void)hipFree( ctx->dsolvy );
+    ctx->dvecs = ctx->dsolvy = nullptr;
+    ctx->dvecs_bytes = ctx->dsolvy_bytes = 0;
+    ctx->wide_refused = SIZE_MAX;
+}
+
+// Whether the two vectors of a pass of nr columns fit beside the factor (option
+// solve_wide_mb: and in how much).  Where they do not, all of the scratch is
+// left to the narrower passes.
+template <typename T>
+bool
+wide_fits( pxd_ctx_t *ctx, int nr )
+{
+    const size_t need = (size_t)ctx->n * nr * sizeof( T );
+    if ( need >= ctx->wide_refused || ( ctx->solve_wide_mb > 0. && 2. * need > ctx->solve_wide_mb * 1048576. ) ) {
+        return false;
+    }
+    if ( grow( &ctx->dvecs, &ctx->dvecs_bytes, need ) || grow( &ctx->dsolvy, &ctx->dsolvy_bytes, need ) ) {
+        drop_vectors( ctx );
+        ctx->wide_refused = need;
+        return false;
+    }
+    return true;
+}
+
+// One wide pass: nq <= NR columns of v (wide_fits).
 template <typename TV, typename T, int NR>
 int
 wide_pass( pxd_ctx_t *ctx, TV *v, int64_t ld, int nq, bool swap )
 {
-    const size_t need = (size_t)ctx->n * NR * sizeof( T );
-    if ( ctx->dvecs_bytes < need ) {
-        if ( ctx->dvecs ) PXD_CHECK( hipFree( ctx->dvecs ) );
-        ctx->dvecs       = nullptr;
-        ctx->dvecs_bytes = 0;
-        PXD_CHECK( hipMalloc( &ctx->dvecs, need ) );
-        ctx->dvecs_bytes = need;
-    }
-    if ( ctx->dsolvy_bytes < need ) {
-        if ( ctx->dsolvy ) PXD_CHECK( hipFree( ctx->dsolvy ) );
-        ctx->dsolvy       = nullptr;
-        ctx->dsolvy_bytes = 0;
-        PXD_CHECK( hipMalloc( &ctx->dsolvy, need ) );
-        ctx->dsolvy_bytes = need;
-    }
     T   *X = (T *)ctx->dvecs, *Y = (T *)ctx->dsolvy;
     auto sweeps = [&] { return wide_sweeps<T, NR>( ctx, X, Y, nq, swap ); };
     hipLaunchKernelGGL( ( k_svw_pack<T, TV, NR> ), dim3( nblocks( ctx->n, 64 ) ), dim3( PXD_THREADS ), 0, ctx->stream,
@@ -1727,16 +1763,20 @@ solve_vectors( pxd_ctx_t *ctx, int64_t nrhs, void *dx, int64_t ldx, int what = S
                void *scr = nullptr )
 {
     int rc = 0;
-    // Wide passes of 32, 16 and 4 columns where they are the faster ones, the
-    // rest by the narrow ones below, which also keep the sweeps on their own,
+    // Wide passes of 32, 16 and 4 columns where they are the faster ones and
+    // their scratch fits, the rest by the narrow ones below, which also keep the sweeps on their own,
     // the Schur parts, the scalar kernels and the allocation-free solve.
     if ( scr == nullptr && what == SOLVE_ALL && ctx->kernels && ctx->schurfcol >= ctx->n ) {
         TV *v = (TV *)dx;
         while ( nrhs > 0 && nrhs >= wide_from<T>( ctx ) && rc == 0 ) {
-            const int nq = (int)std::min<int64_t>( nrhs, 32 );
-            rc = nq > 16  ? wide_pass<TV, T, 32>( ctx, v, ldx, nq, swap )
-                 : nq > 4 ? wide_pass<TV, T, 16>( ctx, v, ldx, nq, swap )
-                          : wide_pass<TV, T, 4>( ctx, v, ldx, nq, swap );
+            int nr = nrhs > 16 ? 32 : nrhs > 4 ? 16 : 4;
+            if ( !wide_fits<T>( ctx, nr ) && ( nr != 32 || !wide_fits<T>( ctx, nr = 16 ) ) ) {
+                break;
+            }
+            const int nq = (int)std::min<int64_t>( nrhs, nr );
+            rc = nr == 32   ? wide_pass<TV, T, 32>( ctx, v, ldx, nq, swap )
+                 : nr == 16 ? wide_pass<TV, T, 16>( ctx, v, ldx, nq, swap )
+                            : wide_pass<TV, T, 4>( ctx, v, ldx, nq, swap );
             v += nq * ldx;
             nrhs -= nq;
         }
@@ -1776,10 +1816,8 @@ solve_vectors( pxd_ctx_t *ctx, int64_t nrhs, void *dx, int64_t ldx, int what = S
         T *xs = (T *)scr;
         T *ys = nullptr;
         if ( scr == nullptr ) {
-            if ( ctx->dvecs_bytes < need ) {
-                if ( ctx->dvecs ) PXD_CHECK( hipFree( ctx->dvecs ) );
-                PXD_CHECK( hipMalloc( &ctx->dvecs, need ) );
-                ctx->dvecs_bytes = need;
+            if ( ( rc = grow_or_say( &ctx->dvecs, &ctx->dvecs_bytes, need ) ) != 0 ) {
+                return rc;
             }
             xs = (T *)ctx->dvecs;
         }
@@ -2106,6 +2144,15 @@ pxd_set_option( pxd_ctx_t *ctx, const char *key, double value )
             return 7;
         }
         ctx->solve_wide_rhs = (int)value;
+        return 0;
+    }
+    if ( k == "solve_wide_mb" ) {
+        if ( !( value >= 0. ) ) {
+            return 7;
+        }
+        ctx->solve_wide_mb = value;
+        PXD_CHECK( hipSetDevice( ctx->device ) );
+        drop_vectors( ctx );
         return 0;
     }
     if ( k == "solve_split_max" || k == "solve_split_wg" ) {
@@ -2451,11 +2498,13 @@ pxd_factorize( pxd_ctx_t *ctx, int factotype, int factor_flttype, double thresho
         // matrix-core kernels
         return 7;
     }
+    ctx->wide_refused = SIZE_MAX;
     const bool lu    = ( factotype == FACT_GETRF );
     size_t     es    = elt_size( factor_flttype );
     size_t     bytes = std::max<int64_t>( ctx->coefnbr, 1 ) * es;
     size_t     dinvb = std::max<int64_t>( ctx->dinvnbr, 1 ) * es;
     if ( ctx->dL == nullptr || ctx->coef_bytes != bytes || ctx->fflt != factor_flttype ) {
+        drop_vectors( ctx );   // the solves' scratch must not keep a factor from fitting
         void *old[] = { ctx->dL, ctx->ddinv, ctx->dU, ctx->dudinv };
         for ( void *q : old ) {
             if ( q ) PXD_CHECK( hipFree( q ) );

@@ -56,3 +56,27 @@ def test_wide_passes_match_narrow_passes(kind, facto, mixed, edges):
     with pytest.raises(px.PastixError):
         px.set_option(pd, "solve_wide_rhs", 0)
     px.finalize(pd)
+
+
+@pytest.mark.parametrize("kind,facto,mixed,edges", [CASES[0], CASES[1], CASES[5], CASES[6]])
+def test_blocks_whose_scratch_does_not_fit_are_taken_narrower(kind, facto, mixed, edges):
+    """solve_wide_mb below the scratch of 32, of 16 and of 4 columns, set in
+    between solves: the same path as where the device has no room."""
+    spm = make_problem(kind, *edges, dof=1)
+    pd, iparm, dparm = analyzed(spm, *edges, facto=facto, mixed=mixed)
+    px.task_numfact(pd, spm)
+    eps = np.finfo(np.float32 if mixed else np.float64).eps
+    mb = 2 * spm.n * np.dtype(np.float32 if mixed else np.float64).itemsize / 2 ** 20   # of one column
+    mb *= 2 if spm.is_complex else 1
+    _, b = spm.gen_rhs(37, seed=1)
+    px.set_option(pd, "solve_wide_rhs", 1e9)
+    want = _solve(pd, b, 0)
+    px.set_option(pd, "solve_wide_rhs", 1)
+    for columns in (33, 31, 15, 3, 17, 0):
+        px.set_option(pd, "solve_wide_mb", columns * mb)
+        for rep in range(2):   # captured and replayed
+            got = _solve(pd, b, 0)
+            assert np.abs(got - want).max() <= 200 * eps * np.abs(want).max(), (columns, rep)
+    with pytest.raises(px.PastixError):
+        px.set_option(pd, "solve_wide_mb", -1)
+    px.finalize(pd)
