@@ -2140,7 +2140,7 @@ pxd_set_option( pxd_ctx_t *ctx, const char *key, double value )
         return 0;
     }
     if ( k == "solve_wide_rhs" ) {
-        if ( value < 1. || value > 1e9 ) {
+        if ( !( value == 0. || ( value >= 1. && value <= 1e9 ) ) ) {   // 0: back to the rule
             return 7;
         }
         ctx->solve_wide_rhs = (int)value;

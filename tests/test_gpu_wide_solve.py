@@ -53,8 +53,12 @@ def test_wide_passes_match_narrow_passes(kind, facto, mixed, edges):
         px.set_option(pd, "solve_wide_rhs", 1)
         got = _solve(pd, b, trans)
         assert np.abs(got - want).max() <= 200 * eps * np.abs(want).max(), (nrhs, trans, small, graph)
-    with pytest.raises(px.PastixError):
-        px.set_option(pd, "solve_wide_rhs", 0)
+        px.set_option(pd, "solve_wide_rhs", 0)   # back to the default rule
+        got = _solve(pd, b, trans)
+        assert np.abs(got - want).max() <= 200 * eps * np.abs(want).max(), (nrhs, trans, small, graph)
+    for value in (-1, 0.5, 2e9):
+        with pytest.raises(px.PastixError):
+            px.set_option(pd, "solve_wide_rhs", value)
     px.finalize(pd)
 
 
