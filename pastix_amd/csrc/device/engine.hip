@@ -1997,8 +1997,10 @@ load_tuning( pxd_ctx_t *ctx )
     if ( f == nullptr ) {
         return;
     }
-    char line[256];
-    while ( fgets( line, sizeof( line ), f ) ) {
+    // whole lines, however long: the rest of a cut comment would be read as an option
+    char  *line = nullptr;
+    size_t cap  = 0;
+    while ( getline( &line, &cap, f ) > 0 ) {
         char  *hash = strchr( line, '#' );
         char   key[128];
         double value;
@@ -2009,6 +2011,7 @@ load_tuning( pxd_ctx_t *ctx )
             fprintf( stderr, "pastix_amd device: %s: unknown option %s\n", path.c_str(), key );
         }
     }
+    free( line );
     fclose( f );
     ctx->tuning_file = path;
 }

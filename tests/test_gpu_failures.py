@@ -12,7 +12,9 @@ every kernel still exits normally:
   matrix as well, sopalin/coeftab.c);
 - IPARM_ITERMAX = 1: the refinement stops after one iteration, short of
   the target, and reports that iteration count (reference
-  refinement/z_refine_gmres.c:75, :314 stop on itermax)."""
+  refinement/z_refine_gmres.c:75, :314 stop on itermax);
+- a tuning file with comments longer than any buffer and with an unknown
+  key: the key is reported, the comments are not."""
 import ctypes
 
 import numpy as np
@@ -77,3 +79,16 @@ def test_refinement_stops_at_itermax():
     assert berr1 < berr0          # one iteration helps ...
     assert berr1 > 1e-15          # ... but a single-precision factor needs more
     px.finalize(pd)
+
+
+def test_tuning_file_lines_are_read_whole(tmp_path, monkeypatch, capfd):
+    path = tmp_path / "tuning.txt"
+    comments = ["#" + "x" * n + " not_an_option 5\n" for n in (100, 254, 255, 600)]
+    path.write_text("".join(comments) + "upd_big_rows 48  # " + "y" * 300 + "\nno_such_option 3\n")
+    monkeypatch.setenv("PXD_TUNING_FILE", str(path))
+    spm = px.Spm.laplacian7(6, 6, 6)
+    pd, iparm, dparm = analyzed(spm, 6)
+    px.task_numfact(pd, spm)
+    px.finalize(pd)
+    err = capfd.readouterr().err
+    assert err.count("unknown option") == 1 and "unknown option no_such_option" in err
