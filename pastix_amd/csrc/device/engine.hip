@@ -103,6 +103,7 @@ struct pxd_ctx_s {
     // structure
     int64_t n = 0, cblknbr = 0, bloknbr = 0, coefnbr = 0, dinvnbr = 0;
     int32_t colmax = 0;
+    int64_t cblk_entries = 0;   // of the largest cblk
     std::vector<dcblk> hcb;
     std::vector<dblok> hbk;
     dcblk   *dcb = nullptr;
@@ -2359,9 +2360,12 @@ pxd_set_structure( pxd_ctx_t *ctx, int64_t n, int64_t cblknbr, int64_t bloknbr,
     }
     ctx->dinvnbr = dinv;
     // the update kernels address a cblk's coefficients with 32-bit byte
-    // offsets (buffer loads): every cblk must stay below 2 GiB in double
+    // offsets, of which those from PXD_OOB (2 GiB) on mean none: every cblk
+    // must stay below 2 GiB in double (complex double: pxd_factorize)
+    ctx->cblk_entries = 0;
     for ( int64_t k = 0; k < cblknbr; k++ ) {
         const dcblk &c = ctx->hcb[k];
+        ctx->cblk_entries = std::max( ctx->cblk_entries, (int64_t)c.stride * ( c.lcolnum - c.fcolnum + 1 ) );
         if ( (double)c.stride * ( c.lcolnum - c.fcolnum + 1 ) * 8. >= 2147483648. ) {
             fprintf( stderr, "pastix_amd device: cblk %lld holds more than 2 GiB of coefficients\n", (long long)k );
             return 3;
@@ -2500,6 +2504,11 @@ pxd_factorize( pxd_ctx_t *ctx, int factotype, int factor_flttype, double thresho
         // LU of a general matrix needs its transpose for the U side, and the
         // matrix-core kernels
         return 7;
+    }
+    if ( ctx->cblk_entries >= ( (int64_t)1 << 31 ) / (int64_t)elt_size( factor_flttype ) ) {
+        fprintf( stderr, "pastix_amd device: a cblk holds %lld entries, more than 2 GiB of coefficients\n",
+                 (long long)ctx->cblk_entries );
+        return 3;
     }
     ctx->wide_refused = SIZE_MAX;
     const bool lu    = ( factotype == FACT_GETRF );

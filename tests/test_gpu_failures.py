@@ -13,6 +13,8 @@ every kernel still exits normally:
 - IPARM_ITERMAX = 1: the refinement stops after one iteration, short of
   the target, and reports that iteration count (reference
   refinement/z_refine_gmres.c:75, :314 stop on itermax);
+- a column block of 2 GiB in complex double, beyond the kernels' 32-bit byte
+  offsets: refused before anything is allocated;
 - a tuning file with comments longer than any buffer and with an unknown
   key: the key is reported, the comments are not."""
 import ctypes
@@ -92,3 +94,39 @@ def test_tuning_file_lines_are_read_whole(tmp_path, monkeypatch, capfd):
     px.finalize(pd)
     err = capfd.readouterr().err
     assert err.count("unknown option") == 1 and "unknown option no_such_option" in err
+
+
+def test_column_block_of_two_gib_is_refused():
+    """One cblk of 320 columns whose rows face 1199 cblks of 350: 2^27 entries
+    and more, 2 GiB at 16 bytes each."""
+    n0, w, m = 320, 350, 1199
+    n = n0 + w * m
+    assert n0 * n * 16 >= 2 ** 31 > n0 * n * 8
+    first = np.concatenate([[0], n0 + w * np.arange(m)])
+    last = np.concatenate([[n0 - 1], first[2:] - 1, [n - 1]])
+    cblk = np.zeros((m + 2, 6), dtype=np.int64)
+    cblk[:-1, 0], cblk[:-1, 1], cblk[-1, :2] = first, last, n
+    cblk[:, 2] = np.concatenate([[0], np.arange(m + 1) + m + 1])        # first bloks: 1 + m, then one each
+    cblk[:, 3] = np.concatenate([[n], np.full(m, w), [0]])
+    cblk[:, 4] = np.concatenate([[0], n0 * n + w * w * np.arange(m + 1)])
+    cblk[:, 5] = np.concatenate([[0, 0], np.arange(1, m + 1)])
+    k = np.arange(1, m + 1)
+    blok = np.zeros((2 * m + 2, 5), dtype=np.int64)
+    blok[:m + 1, 0], blok[:m + 1, 1], blok[:m + 1, 3], blok[:m + 1, 4] = first, last, np.arange(m + 1), first * n0
+    blok[m + 1:-1, 0], blok[m + 1:-1, 1], blok[m + 1:-1, 2], blok[m + 1:-1, 3] = first[1:], last[1:], k, k
+    browtab = np.arange(1, m + 1, dtype=np.int64)
+    lib, vp, ll = px.lib, ctypes.c_void_p, ctypes.c_int64
+    ctx = vp()
+    lib.pxd_set_structure.argtypes = [vp, ll, ll, ll, vp, vp, vp, ll]
+    lib.pxd_set_matrix.argtypes = [vp, ctypes.c_int, ctypes.c_int, ll, ll] + [vp] * 6
+    lib.pxd_factorize.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_double, vp]
+    px._check("pxd_create", lib.pxd_create(ctypes.byref(ctx), 0))
+    px._check("pxd_set_structure", lib.pxd_set_structure(ctx, n, m + 1, 2 * m + 1, cblk.ctypes.data, blok.ctypes.data,
+                                                         browtab.ctypes.data, int(cblk[-1, 4])))
+    colptr, rows, values = np.arange(n + 1, dtype=np.int64), np.arange(n, dtype=np.int64), np.ones(n, np.complex128)
+    px._check("pxd_set_matrix", lib.pxd_set_matrix(ctx, px.SpmComplex64, px.PastixSymmetric, n, n, colptr.ctypes.data,
+                                                   rows.ctypes.data, values.ctypes.data, None, None, None))
+    npiv = ll()
+    assert lib.pxd_factorize(ctx, px.PastixFactLDLT, px.SpmComplex64, 1e-10,
+                             ctypes.byref(npiv)) == px.PASTIX_ERR_NOTIMPLEMENTED
+    lib.pxd_destroy(ctx)
