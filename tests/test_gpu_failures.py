@@ -24,7 +24,7 @@ import pytest
 
 import pastix_amd as px
 import oracle_ref as orc
-from helpers import analyzed, cblk_diff, static_pivot_threshold
+from helpers import analyzed, cblk_diff, make_problem, static_pivot_threshold
 
 pytestmark = pytest.mark.gpu
 
@@ -45,6 +45,39 @@ def test_panel_wait_bound_gives_up_and_reports_internal_error():
     L = px.get_coeftab(pd, s["coefnbr"], np.float64)
     F = orc.OracleFactor(s, px.bcsc_export(pd), static_pivot_threshold(dparm, np.float64))
     assert cblk_diff(s, L, F.L, np.float64) <= 10.0
+    px.finalize(pd)
+
+
+@pytest.mark.parametrize("kind,facto,mixed,nx", [("lap7", px.PastixFactPOTRF, 1, 20),
+                                                 ("lap7sd", px.PastixFactLDLT, 0, 14),
+                                                 ("lap7sd", px.PastixFactLDLT, 1, 14),
+                                                 ("helmholtz7", px.PastixFactLDLT, 0, 14),
+                                                 ("helmholtz7", px.PastixFactLDLT, 1, 14),
+                                                 ("convdiff27", px.PastixFactLU, 0, 11),
+                                                 ("convdiff27", px.PastixFactLU, 1, 11),
+                                                 ("helmholtz7", px.PastixFactLU, 0, 11),
+                                                 ("helmholtz7", px.PastixFactLU, 1, 11)])
+def test_every_panel_gives_up_and_recovers(kind, facto, mixed, nx):
+    """The same for the other factorizations and arithmetics (LU: both sides'
+    rows and inverse columns wait)."""
+    spm = make_problem(kind, nx)
+    pd, iparm, dparm = analyzed(spm, nx, facto=facto, mixed=mixed)
+    try:
+        px.set_option(pd, "wait_ms", 0)
+        with pytest.raises(px.PastixError) as e:
+            px.task_numfact(pd, spm)
+        assert e.value.code == px.PASTIX_ERR_INTERNAL
+    finally:
+        px.set_option(pd, "wait_ms", 2000)
+    px.task_numfact(pd, spm)
+    dtype = {(0, 0): np.float64, (0, 1): np.float32, (1, 0): np.complex128, (1, 1): np.complex64}[int(spm.is_complex), mixed]
+    s = px.solver_export(pd)
+    oracle = {px.PastixFactPOTRF: orc.OracleFactor, px.PastixFactLDLT: orc.OracleLDLT, px.PastixFactLU: orc.OracleLU}
+    F = oracle[facto](s, px.bcsc_export(pd, complex_=spm.is_complex), static_pivot_threshold(dparm, dtype), dtype)
+    full = facto != px.PastixFactPOTRF
+    assert cblk_diff(s, px.get_coeftab(pd, s["coefnbr"], dtype), F.L, dtype, full_diag=full) <= 10.0
+    if facto == px.PastixFactLU:
+        assert cblk_diff(s, px.get_coeftab(pd, s["coefnbr"], dtype, side=1), F.U, dtype, full_diag=True) <= 10.0
     px.finalize(pd)
 
 

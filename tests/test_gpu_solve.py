@@ -1,8 +1,9 @@
 """The level-by-level solve sweeps against the oracle's solve with the
 device's own factor, for every factorization, arithmetic and precision
 (double and single factors, real and complex; Cholesky, LDL^T and LU), with
-right-hand side counts that take one pass and several (20 RHS: passes of 8),
-with the passes replayed from captured graphs (engine option solve_graph =
+right-hand side counts that take one pass and several, by the default rule
+(these systems: wide passes of 4, 16 and 32) and in narrow passes of 8
+(engine option solve_wide_rhs = 1e9), with the passes replayed from captured graphs (engine option solve_graph =
 1, the default) and launched kernel by kernel (0); and the graph-replayed
 solve against the same sweeps launched one by one, replay after replay,
 with other device work in between.
@@ -43,8 +44,9 @@ def _problem(kind, nx):
 
 @pytest.mark.parametrize("graph", [1, 0])
 @pytest.mark.parametrize("nrhs", [1, 4, 20])
+@pytest.mark.parametrize("wide_rhs", [0, 1e9])
 @pytest.mark.parametrize("kind,facto,mixed,nx", CASES)
-def test_level_solve_matches_oracle_solve(kind, facto, mixed, nx, nrhs, graph):
+def test_level_solve_matches_oracle_solve(kind, facto, mixed, nx, wide_rhs, nrhs, graph):
     """The device solve (graph-replayed passes or launched kernel by kernel)
     against the oracle's supernodal solve with the device's own factor, in
     the factor precision (a single factor: vectors rounded to single, as the
@@ -52,6 +54,7 @@ def test_level_solve_matches_oracle_solve(kind, facto, mixed, nx, nrhs, graph):
     spm = _problem(kind, nx)
     pd, iparm, dparm = analyzed(spm, nx, facto=facto, mixed=mixed)
     px.set_option(pd, "solve_graph", graph)
+    px.set_option(pd, "solve_wide_rhs", wide_rhs)
     px.task_numfact(pd, spm)
     x0, b = spm.gen_rhs(nrhs, seed=3)
     x = np.array(b, order="F", copy=True)
@@ -103,18 +106,20 @@ def test_solve_on_a_refactorized_instance():
     px.finalize(pd2)
 
 
+@pytest.mark.parametrize("wide_rhs", [0, 1e9])
 @pytest.mark.parametrize("kind,facto,mixed,nx", [("lap7", None, 0, 10), ("lap7", None, 1, 10),
                                                  ("helm", px.PastixFactLDLT, 0, 8),
                                                  ("convdiff27", px.PastixFactGETRF, 1, 8)])
-def test_graph_solve_replays_match_eager(kind, facto, mixed, nx):
-    """Captured passes (8 and then 3 columns: two graphs) replayed five
-    times; between replays the same sweeps run eagerly (solve_graph = 0),
+def test_graph_solve_replays_match_eager(kind, facto, mixed, nx, wide_rhs):
+    """Captured passes (one wide pass of 11 columns; narrow, 8 and then 3
+    columns: two graphs) replayed five times; between replays the same sweeps run eagerly (solve_graph = 0),
     and a refactorization in the middle rebuilds the task lists, after which
     the graphs are captured again.  Every replay agrees with the eager solve
     to rounding (atomic accumulation) and with it meets the backward error of
     the factor precision."""
     spm = _problem(kind, nx)
     pd, iparm, dparm = analyzed(spm, nx, facto=facto, mixed=mixed)
+    px.set_option(pd, "solve_wide_rhs", wide_rhs)
     px.task_numfact(pd, spm)
     eps = np.finfo(np.float32 if mixed else np.float64).eps
     for rep in range(5):

@@ -1,6 +1,8 @@
 """Every blok update on the tall tiles whose operands go straight into LDS
-(upd_big_rows = 1, upd_small = 0), for every factorization and arithmetic,
-against the oracle tile by tile.  The grids have ragged edges: source cblks
+(upd_big_rows = 1, upd_small = 0), and on those whose operands go through
+registers (upd_dma = 0), for every factorization and arithmetic, against the
+oracle tile by tile; in float also with more LDS per workgroup (upd_dma_pad,
+which the other types do not take).  The grids have ragged edges: source cblks
 of 1 to 306 columns (stages that end inside their k values), facing bloks
 narrower and wider than the 64 columns of a tile, row tiles that end inside
 a wave's rows, and sources that add to the same columns (atomic tiles)."""
@@ -23,13 +25,14 @@ CASES = [("lap7", px.PastixFactPOTRF, np.float64, (20, 17, 18)), ("lap7", px.Pas
          ("helmholtz7", px.PastixFactLU, np.complex64, (11, 12, 13))]
 
 
-@pytest.mark.parametrize("pad", [0, 8192])
-@pytest.mark.parametrize("kind,facto,dtype,edges", CASES)
-def test_every_update_on_the_tall_tiles_matches_oracle(kind, facto, dtype, edges, pad):
+@pytest.mark.parametrize("kind,facto,dtype,edges,dma,pad",
+                         [c + (dma, 0) for c in CASES for dma in (1, 0)] +
+                         [c + (1, 8192) for c in CASES if c[2] is np.float32])
+def test_every_update_on_the_tall_tiles_matches_oracle(kind, facto, dtype, edges, dma, pad):
     spm = make_problem(kind, *edges)
     mixed = int(np.dtype(dtype) in (np.float32, np.complex64))
     pd, iparm, dparm = analyzed(spm, *edges, facto=facto, mixed=mixed)
-    for key, value in (("upd_big_rows", 1), ("upd_small", 0), ("upd_dma", 1), ("upd_dma_pad", pad)):
+    for key, value in (("upd_big_rows", 1), ("upd_small", 0), ("upd_dma", dma), ("upd_dma_pad", pad)):
         px.set_option(pd, key, value)
     px.task_numfact(pd, spm)
     s = px.solver_export(pd)
