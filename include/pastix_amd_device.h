@@ -102,7 +102,8 @@ int  pxd_get_stats( const pxd_ctx_t *ctx, pxd_stats_t *stats );
  *   "solve_graph"   1: each solve pass replays the sweeps' launches from a
  *                   graph captured on first use (default); 0: launched one by one
  *   "solve_wide_max" level-solve launches with at least this many tiles load
- *                   16 columns per batch (default 128)
+ *                   16 columns per batch and share no tile (default 128; the
+ *                   blocks of solve_wide_rhs take the sharing from it alone)
  *   "solve_wide_rhs" fewest right-hand sides that a solve takes in blocks of
  *                   4, 16 or 32 on the matrix cores; 0 (default): the
  *                   measured rule (double: 1; single: 5, fewer on small
@@ -116,7 +117,9 @@ int  pxd_get_stats( const pxd_ctx_t *ctx, pxd_stats_t *stats );
  *   "solve_spread"  cblks with at least this many 64-row tiles (default 16;
  *                   0: none) gather the backward sweep's sums in 8 partial
  *                   copies instead of atomics into one; the records follow
- *                   at the next factorization, 0 takes effect at once
+ *                   at the next factorization, 0 takes effect at once.  The
+ *                   narrow passes alone (large single factors with up to 4
+ *                   right-hand sides, the Schur solves, solve_wide_rhs)
  *   "solve_split_max", "solve_split_wg"  smaller launches share each tile
  *                   among up to solve_split_max workgroups (default 4),
  *                   solve_split_wg workgroups in all (default 512)

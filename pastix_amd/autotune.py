@@ -12,16 +12,21 @@ rounding:
   for updates of at most upd_small_m rows, upd_small_n columns and 32 k
   values;
 - ``solve_wide_max``: level-solve launches from which the tiles load 16
-  columns per batch instead of all of them;
+  columns per batch instead of all of them and share no tile (the wide
+  passes of double and small factors take the sharing from it alone);
 - ``panel_mw``: the multi-workgroup panel (0: Cholesky by one workgroup);
 - ``upd_dma``: tall tiles on the kernel that loads its operands straight
   into LDS;
-- ``upd_dma_pad``: extra LDS per workgroup of that kernel, which sets how
-  many of its workgroups share a CU with the lookahead stream's panels;
+- ``upd_dma_pad``: extra LDS per workgroup of that kernel in single
+  precision, which sets how many of its workgroups share a CU with the
+  lookahead stream's panels;
 - ``solve_split_max``, ``solve_split_wg``: how many workgroups share a tile
   of a level-solve launch with few tiles;
 - ``solve_spread``: the fewest tiles of a cblk whose backward gather goes
-  through partial-sum copies (0: none).
+  through partial-sum copies in the narrow passes (0: none).
+
+``solve_wide_rhs``, from which right-hand sides go in wide passes, is not
+searched: its default is a rule by type and size.
 
 The search is coordinate descent from the current values (each option in
 turn over its candidates, the others fixed, two passes); the objective is

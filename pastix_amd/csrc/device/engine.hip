@@ -1739,8 +1739,10 @@ wide_pass( pxd_ctx_t *ctx, TV *v, int64_t ld, int nq, bool swap )
 
 // Fewest right-hand sides for which a wide pass is the faster one (measured,
 // narrow against wide, ms): in double always (100^3: 5.80 / 5.22 for 1 and
-// 9.7 / 5.8 for 8; 41^3 LU 0.59 / 0.51 for 1; 15^3 complex 0.154 / 0.142); in
-// single from 5 on (100^3: 4.14 / 4.92 for 4, 5.48 / 4.80 for 5), and always on
+// 9.7 / 5.8 for 8; 41^3 LU 0.59 / 0.51 for 1; complex LDL^T 15^3 0.154 / 0.142,
+// 50^3 1.55 / 1.51, LU 42^3 1.04 / 1.01 for 1, 1.98 / 1.06 for 8); in
+// single from 5 on (100^3: 4.14 / 4.92 for 4, 5.48 / 4.80 for 5; complex 80^3:
+// 3.81 / 4.70 for 4, 6.31 / 4.76 for 5, 10.75 / 5.27 for 12), and always on
 // small factors, which are all latency: real ones (40^3, 95 MB: 0.455 / 0.436
 // for 1; 50^3, 245 MB: 0.698 / 0.701 for 4; 41^3 LU, 235 MB: 0.484 / 0.509 for
 // 1), and complex ones, four products for each, only while they are tiny (15^3,

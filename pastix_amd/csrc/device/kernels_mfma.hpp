@@ -317,7 +317,7 @@ k_potrf2( const int32_t *__restrict__ list, const dcblk *__restrict__ cb, T *__r
 // (cblk, block column J).  The diagonal blocks D_K = L[K,K]^{-1} were written
 // to Linv by the panel.  Column sweep: R = -L[J+1:, J] D_J, then for K = J+1,
 // J+2, ...: X[K,J] = D_K R[K], R[K+1:] -= L[K+1:, K] X[K,J].  The first rcap
-// rows of R stay in LDS, the rest (wide cblks in complex double) in place in
+// rows of R stay in LDS, rows that would not fit in place in
 // Linv, where X[K,J] later overwrites them; both products run on the matrix
 // cores.
 template <typename T>
@@ -1199,11 +1199,16 @@ k_update_big( const upd_task *__restrict__ tasks, int32_t ntasks, const dcblk *_
 // slabs 65.3 ms.  The rows' places in the facing cblk are in the registers of
 // the lanes that loaded them.
 //
-// What bounds it: the read-modify-write of C beside the products.  100^3,
-// update launches alone: float 66.7 -> 65.3 ms against the same scheme with
-// two workgroup barriers per slab and no load in flight across a stage's
-// barrier, double 136.2 -> 133.2 ms and 80^3 complex64 LDL^T 73.0 -> 71.8 ms
-// against k_update_big (factorizations 155.8 -> 150.7 and 88.0 -> 84.9 ms).
+// What bounds it: the matrix cores (busy 0.71 of the time in float, 0.73 in
+// double), and the movement of the operands beside them.  100^3 double, update
+// launches alone, 126 ms: timing-only copies without the loop's loads 108.9,
+// without the C part 121.4, without both 101.2; the products alone take 96 at
+// the rate of a large matrix product.  Several pieces of a supernode updating
+// C together, which halves the bytes of C, gained nothing.  Float 66.7 -> 65.3
+// ms against the same scheme with two workgroup barriers per slab and no load
+// in flight across a stage's barrier, double 136.2 -> 133.2 ms and 80^3
+// complex64 LDL^T 73.0 -> 71.8 ms against k_update_big (factorizations 155.8
+// -> 150.7 and 88.0 -> 84.9 ms).
 //
 // LDL^T scales A by D (kept in LDS), the reference's D L^T workspace.
 

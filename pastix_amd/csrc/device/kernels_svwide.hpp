@@ -5,11 +5,15 @@
 // The sweeps of kernels_svsolve.hpp carry at most 8 right-hand sides per
 // pass over the factor, so a block of 32 streamed it four times, and each
 // level's launches took their 10 to 20 us of dependent memory trips four
-// times.  Here a pass carries NR = 16 or 32: a factor entry is one operand of
-// a 16 x 16 x 4 product instead of 8 multiply-adds with 8 LDS reads.  The
+// times.  Here a pass carries NR = 4, 16 or 32: a factor entry is one operand
+// of a 16 x 16 x 4 product instead of 8 multiply-adds with 8 LDS reads.  The
 // vectors are held by rows, NR values of a row next to each other (V[row *
 // NR + q]), so that every operand row, result and atomic is one contiguous
-// run of 16 values; the columns q >= nq of a pass hold zeros.
+// run of min(NR, 16) values; the columns q >= nq of a pass hold zeros.  With NR
+// = 4 the lanes 4 .. 15 of a product's columns repeat the last one and their
+// results are dropped: a quarter of the product counts, which a pass over a
+// double factor can afford and one over a large single factor cannot
+// (wide_from in engine.hip).
 //
 // Bound: the factor's bytes on the wide levels (each entry once per sweep),
 // the three or four dependent trips of a level's two launches at the top.
