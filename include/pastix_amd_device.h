@@ -178,7 +178,9 @@ int pxd_set_matrix( pxd_ctx_t *ctx, int flttype, int mtxtype, int64_t n, int64_t
  * SYTRF.  factor_flttype: SpmDouble/SpmFloat for real matrices, SpmComplex64/
  * SpmComplex32 for complex ones (single = mixed precision).  |pivot| <
  * threshold is replaced by threshold (static pivoting); the number of such
- * replacements is returned in *nbpivots.
+ * replacements is returned in *nbpivots.  A cblk of 2 GiB or more in the
+ * factor's type is refused (PASTIX_ERR_NOTIMPLEMENTED), as is one wider than
+ * the kernels take.
  */
 int pxd_factorize( pxd_ctx_t *ctx, int factotype, int factor_flttype,
                    double threshold, int64_t *nbpivots );

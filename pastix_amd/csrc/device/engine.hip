@@ -1552,8 +1552,7 @@ drop_solve_graphs( pxd_ctx_t *ctx )
 }
 
 // Whether the sweeps of a pass run as a captured graph: the full solve of
-// the matrix-core path without the one-launch sweeps (their pass counters
-// change from call to call) and without a Schur part.
+// the matrix-core path without a Schur part.
 bool
 graph_ok( const pxd_ctx_t *ctx, int what, bool swap )
 {
